@@ -206,6 +206,7 @@ struct OrderedArgs {
   int64_t ld;           // jbuf row stride in events: n rounded up to a 16-event tile, so that
                         // every tile of a colour row is whole 128-byte lines
   int h0, nhel;         // helicity rows h0 .. h0+nhel-1 (or 1 row for an explicit vector)
+  int cparts, cper;     // orderings in cparts ranges of cper (even) each, one per block
   void* jbuf;           // [nhel][NCOLOR][n] complex R
 };
 
@@ -227,6 +228,14 @@ struct OrderedStage {
   static constexpr int NSLOT = NWF + NINV + NFS;
 };
 
+// One block takes 64 events through one set of gluon helicities (its four top / anti-top rows)
+// and one range of the orderings: blockIdx.x = the event tile, blockIdx.y = (gluon helicities,
+// range).  Nothing is shared between gluon helicity sets but the event's invariants and
+// spinors (1-2% of a set's work, computed once more for each), so a call of few events still
+// fills the chip, and a large one ends without a half-empty round of long waves.  Against one
+// wave walking every set of its 64 events: t t~ g g FP64, 1,000 events, 3,117 -> 103 us; t t~ g g g
+// FP32, 257 events, 44.2 -> 0.31 ms, 50,000 events, 42.2 -> 33.7 ms; t t~ g g FP32, 1,048,576
+// events, 37.9 -> 35.2 ms (the momenta no longer stay live across the sets: 244 -> 184 VGPRs).
 template <class T, class R, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) k_ordered_jamps(OrderedArgs a) {
   constexpr int NG = T::NG, NE = T::NEXTERNAL, NC = T::NCOLOR;
@@ -303,6 +312,8 @@ __global__ void __launch_bounds__(BLOCK) k_ordered_jamps(OrderedArgs a) {
   // and every helicity comes from the vector.
   static_assert(T::NCOMB == (4 << NG), "every helicity combination is a row");
   const int r0 = a.h0, r1 = a.h0 + a.nhel;
+  const int g = (r0 >> 2) + (int)blockIdx.y / a.cparts;
+  const int c0 = ((int)blockIdx.y % a.cparts) * a.cper, c1 = c0 + a.cper < NC ? c0 + a.cper : NC;
   constexpr int PRE = NG - 2;
   W<R> J[NG][NG], O[NG];
   cx<R> SD[NG][NG];   // adjacent-range dot sums S(a..b) of the four-gluon terms
@@ -315,135 +326,132 @@ __global__ void __launch_bounds__(BLOCK) k_ordered_jamps(OrderedArgs a) {
   // ap) and the top-line denominators rt (above); pp of the prefix pairs carries over to
   // the second ordering of a pair
   R pp[NG][NG], tp[NG], ap[NG], rt[NG];
+  unsigned hbg = 0u;
+#pragma unroll
+  for (int s = 0; s < NG; ++s) hbg |= ((unsigned)(g >> s) & 1u) << T::gluon_leg(s);
+  const int* helv = a.s.use_helv ? a.s.helv : nullptr;
+#pragma unroll
+  for (int s = 0; s < NG; ++s) {
+    W<R> gw;
+    T::template gluon<R>(p, s, hbg, helv, prm, gw);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      lds[(s * 12 + 2 * q) * BLOCK + t] = gw[q].re;
+      lds[(s * 12 + 2 * q + 1) * BLOCK + t] = gw[q].im;
+    }
+  }
+  // Orderings come in lexicographic order, so orderings 2m and 2m+1 share their first
+  // NG-2 gluons: the currents inside that prefix (J(i..j), j < NG-2) are computed once
+  // per pair and carried to the second ordering.
 #pragma unroll 1
-  for (int g = r0 >> 2; g <= (r1 - 1) >> 2; ++g) {
-    unsigned hbg = 0u;
+  for (int c = c0; c < c1; ++c) {
+    int perm[NG];
 #pragma unroll
-    for (int s = 0; s < NG; ++s) hbg |= ((unsigned)(g >> s) & 1u) << T::gluon_leg(s);
-    const int* helv = a.s.use_helv ? a.s.helv : nullptr;
+    for (int k = 0; k < NG; ++k) perm[k] = T::perm(c, k);
+    const bool fresh = (c & 1) == 0;
 #pragma unroll
-    for (int s = 0; s < NG; ++s) {
-      W<R> gw;
-      T::template gluon<R>(p, s, hbg, helv, prm, gw);
+    for (int k = 0; k < NG; ++k) {
+      if (k < PRE && !fresh) continue;
 #pragma unroll
       for (int q = 0; q < 6; ++q) {
-        lds[(s * 12 + 2 * q) * BLOCK + t] = gw[q].re;
-        lds[(s * 12 + 2 * q + 1) * BLOCK + t] = gw[q].im;
+        J[k][k][q].re = lds[(perm[k] * 12 + 2 * q) * BLOCK + t];
+        J[k][k][q].im = lds[(perm[k] * 12 + 2 * q + 1) * BLOCK + t];
       }
     }
-    // Orderings come in lexicographic order, so orderings 2m and 2m+1 share their first
-    // NG-2 gluons: the currents inside that prefix (J(i..j), j < NG-2) are computed once
-    // per pair and carried to the second ordering.
-#pragma unroll 1
-    for (int c = 0; c < NC; ++c) {
-      int perm[NG];
+    if constexpr (S::NINV > 0) {
+      // the word's pair invariants (the prefix pairs of a pair's second ordering are the
+      // first's), and rt[j] for the top with the first j gluons from the shorter of its
+      // two forms
 #pragma unroll
-      for (int k = 0; k < NG; ++k) perm[k] = T::perm(c, k);
-      const bool fresh = (c & 1) == 0;
+      for (int x = 0; x < NG; ++x) {
+        tp[x] = lds[(S::NWF + T::pair_index(perm[x], NG)) * BLOCK + t];
+        ap[x] = lds[(S::NWF + S::NPI + perm[x]) * BLOCK + t];
 #pragma unroll
-      for (int k = 0; k < NG; ++k) {
-        if (k < PRE && !fresh) continue;
-#pragma unroll
-        for (int q = 0; q < 6; ++q) {
-          J[k][k][q].re = lds[(perm[k] * 12 + 2 * q) * BLOCK + t];
-          J[k][k][q].im = lds[(perm[k] * 12 + 2 * q + 1) * BLOCK + t];
+        for (int y = x + 1; y < NG; ++y) {
+          if (y < PRE && !fresh) continue;
+          pp[x][y] = lds[(S::NWF + T::pair_index(perm[x], perm[y])) * BLOCK + t];
         }
       }
-      if constexpr (S::NINV > 0) {
-        // the word's pair invariants (the prefix pairs of a pair's second ordering are the
-        // first's), and rt[j] for the top with the first j gluons from the shorter of its
-        // two forms
 #pragma unroll
-        for (int x = 0; x < NG; ++x) {
-          tp[x] = lds[(S::NWF + T::pair_index(perm[x], NG)) * BLOCK + t];
-          ap[x] = lds[(S::NWF + S::NPI + perm[x]) * BLOCK + t];
+      for (int j = 1; j < NG; ++j) {
+        // direct: the top and gluons 0..j-1; complementary: the anti-top and gluons j..NG-1
+        const int nd = j + j * (j - 1) / 2, nc = (NG - j) + (NG - j) * (NG - j - 1) / 2;
+        R sd = R(0), md = R(0), sc = R(0), mc = R(0);
 #pragma unroll
-          for (int y = x + 1; y < NG; ++y) {
-            if (y < PRE && !fresh) continue;
-            pp[x][y] = lds[(S::NWF + T::pair_index(perm[x], perm[y])) * BLOCK + t];
+        for (int a = 0; a < j; ++a) {
+          sd += tp[a];
+          md += fabs(tp[a]);
+#pragma unroll
+          for (int b = a + 1; b < j; ++b) {
+            sd += pp[a][b];
+            md += fabs(pp[a][b]);
           }
         }
 #pragma unroll
-        for (int j = 1; j < NG; ++j) {
-          // direct: the top and gluons 0..j-1; complementary: the anti-top and gluons j..NG-1
-          const int nd = j + j * (j - 1) / 2, nc = (NG - j) + (NG - j) * (NG - j - 1) / 2;
-          R sd = R(0), md = R(0), sc = R(0), mc = R(0);
+        for (int a = j; a < NG; ++a) {
+          sc += ap[a];
+          mc += fabs(ap[a]);
 #pragma unroll
-          for (int a = 0; a < j; ++a) {
-            sd += tp[a];
-            md += fabs(tp[a]);
-#pragma unroll
-            for (int b = a + 1; b < j; ++b) {
-              sd += pp[a][b];
-              md += fabs(pp[a][b]);
-            }
+          for (int b = a + 1; b < NG; ++b) {
+            sc += pp[a][b];
+            mc += fabs(pp[a][b]);
           }
+        }
+        rt[j] = nd < nc ? sd : (nc < nd ? sc : (md <= mc ? sd : sc));
+      }
+    }
+    if (fresh) ordered_ranges<NG, 1, PRE, R>(J, SD, pp, prm);
+    ordered_ranges<NG, PRE, NG, R>(J, SD, pp, prm);
+    if constexpr (SHARE_TOP) {
+      // unrolled: OP is indexed by ht
 #pragma unroll
-          for (int a = j; a < NG; ++a) {
-            sc += ap[a];
-            mc += fabs(ap[a]);
+      for (int ht = 0; ht < 2; ++ht) {
+        const int rb = 4 * g + 2 * ht;
+        if (rb + 1 < r0 || rb >= r1) continue;
+        W<R> top, atop;
+        if constexpr (S::NFS > 0) staged_fermion(0, ht, top);
+        else T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG), helv, prm, top, atop);
+        O[0] = top;
+        // O(1..PRE) only involve the prefix gluons: computed once per pair of orderings
+        if (fresh) {
+          ordered_top_line<NG, 1, PRE, R>(O, J, rt, prm);
 #pragma unroll
-            for (int b = a + 1; b < NG; ++b) {
-              sc += pp[a][b];
-              mc += fabs(pp[a][b]);
-            }
-          }
-          rt[j] = nd < nc ? sd : (nc < nd ? sc : (md <= mc ? sd : sc));
+          for (int j = 1; j <= PRE; ++j) OP.o[ht][j] = O[j];
+        } else {
+#pragma unroll
+          for (int j = 1; j <= PRE; ++j) O[j] = OP.o[ht][j];
+        }
+        ordered_top_line<NG, PRE + 1, NG - 1, R>(O, J, rt, prm);
+        const VslashF<R> x = ordered_close_col<NG, R>(O, J);
+#pragma unroll 1
+        for (int ha = 0; ha < 2; ++ha) {
+          const int r = rb + ha;
+          if (r < r0 || r >= r1) continue;
+          if constexpr (S::NFS > 0) staged_fermion(1, ha, atop);
+          else if (ha) T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG) | (1u << T::ATOP_LEG), helv,
+                                               prm, top, atop);
+          jb[((int64_t)(r - r0) * NC + c) * a.ld + el] = ordered_jamp(atop, x, prm);
         }
       }
-      if (fresh) ordered_ranges<NG, 1, PRE, R>(J, SD, pp, prm);
-      ordered_ranges<NG, PRE, NG, R>(J, SD, pp, prm);
-      if constexpr (SHARE_TOP) {
-        // unrolled: OP is indexed by ht
-#pragma unroll
-        for (int ht = 0; ht < 2; ++ht) {
-          const int rb = 4 * g + 2 * ht;
-          if (rb + 1 < r0 || rb >= r1) continue;
-          W<R> top, atop;
-          if constexpr (S::NFS > 0) staged_fermion(0, ht, top);
-          else T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG), helv, prm, top, atop);
-          O[0] = top;
-          // O(1..PRE) only involve the prefix gluons: computed once per pair of orderings
-          if (fresh) {
-            ordered_top_line<NG, 1, PRE, R>(O, J, rt, prm);
-#pragma unroll
-            for (int j = 1; j <= PRE; ++j) OP.o[ht][j] = O[j];
-          } else {
-#pragma unroll
-            for (int j = 1; j <= PRE; ++j) O[j] = OP.o[ht][j];
-          }
-          ordered_top_line<NG, PRE + 1, NG - 1, R>(O, J, rt, prm);
-          const VslashF<R> x = ordered_close_col<NG, R>(O, J);
+    } else {
 #pragma unroll 1
-          for (int ha = 0; ha < 2; ++ha) {
-            const int r = rb + ha;
-            if (r < r0 || r >= r1) continue;
-            if constexpr (S::NFS > 0) staged_fermion(1, ha, atop);
-            else if (ha) T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG) | (1u << T::ATOP_LEG), helv,
-                                                 prm, top, atop);
-            jb[((int64_t)(r - r0) * NC + c) * a.ld + el] = ordered_jamp(atop, x, prm);
-          }
-        }
-      } else {
+      for (int ht = 0; ht < 2; ++ht) {
+        const int rb = 4 * g + 2 * ht;
+        if (rb + 1 < r0 || rb >= r1) continue;
+        W<R> top, atop;
+        if constexpr (S::NFS > 0) staged_fermion(0, ht, top);
+        else T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG), helv, prm, top, atop);
+        O[0] = top;
+        ordered_top_line<NG, 1, NG - 1, R>(O, J, rt, prm);
+        const VslashF<R> x = ordered_close_col<NG, R>(O, J);
 #pragma unroll 1
-        for (int ht = 0; ht < 2; ++ht) {
-          const int rb = 4 * g + 2 * ht;
-          if (rb + 1 < r0 || rb >= r1) continue;
-          W<R> top, atop;
-          if constexpr (S::NFS > 0) staged_fermion(0, ht, top);
-          else T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG), helv, prm, top, atop);
-          O[0] = top;
-          ordered_top_line<NG, 1, NG - 1, R>(O, J, rt, prm);
-          const VslashF<R> x = ordered_close_col<NG, R>(O, J);
-#pragma unroll 1
-          for (int ha = 0; ha < 2; ++ha) {
-            const int r = rb + ha;
-            if (r < r0 || r >= r1) continue;
-            if constexpr (S::NFS > 0) staged_fermion(1, ha, atop);
-            else if (ha) T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG) | (1u << T::ATOP_LEG), helv,
-                                                 prm, top, atop);
-            jb[((int64_t)(r - r0) * NC + c) * a.ld + el] = ordered_jamp(atop, x, prm);
-          }
+        for (int ha = 0; ha < 2; ++ha) {
+          const int r = rb + ha;
+          if (r < r0 || r >= r1) continue;
+          if constexpr (S::NFS > 0) staged_fermion(1, ha, atop);
+          else if (ha) T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG) | (1u << T::ATOP_LEG), helv,
+                                               prm, top, atop);
+          jb[((int64_t)(r - r0) * NC + c) * a.ld + el] = ordered_jamp(atop, x, prm);
         }
       }
     }
@@ -466,16 +474,19 @@ template <class R> struct Vec4;
 template <> struct Vec4<float> { typedef mfx_f32x4 type; };
 template <> struct Vec4<double> { typedef mfx_f64x4 type; };
 
-// |M|^2 of the events of one sub-chunk from their jamps: one wave per 16-event tile,
-// four tiles per block.  Per helicity and tile the matrix cores form D = CF J^T
+// |M|^2 of the events of one sub-chunk from their jamps: one wave per 16-event tile and range
+// of hper helicity rows (blockIdx.y), four tiles per block.  Per helicity and tile the matrix cores form D = CF J^T
 // (NCP x 16: colour rows, event columns) from the integer colour matrix (A operand, in
 // LDS) and the tile's jamps (B operand: lane (i, q) holds J[event i][colour 4 s + q] for
 // every k-step s), then each lane dots its D entries with jamps it already holds.  For
 // that, the colour of A row drow(q, r) of row tile mt is 4 (4 mt + r) + q: the output the
 // lane holds in register r is then the row of the colour of its k-step 4 mt + r, and the
 // jamps are read once.  The four lane quarters of each event are summed at the end.
+// With more than one range of rows (few events: the rows of one tile are then spread over
+// the chip) a wave leaves its 16 sums in place of jamps that it alone has read, colour 0 of
+// its first row, and k_colour_sum adds the ranges in order.
 template <class T, class R>
-__global__ void __launch_bounds__(256) k_colour_mfma(const void* jbuf, int64_t n, int64_t ld, int nhel,
+__global__ void __launch_bounds__(256) k_colour_mfma(void* jbuf, int64_t n, int64_t ld, int nhel, int hper,
                                                      double scale, int accumulate, double* out) {
   constexpr int NC = T::NCOLOR;
   constexpr int NCP = (NC + 15) / 16 * 16;    // padded colour rows of D
@@ -493,6 +504,7 @@ __global__ void __launch_bounds__(256) k_colour_mfma(const void* jbuf, int64_t n
   }
   __syncthreads();
   const cx<R>* J = reinterpret_cast<const cx<R>*>(jbuf);
+  const int h0 = (int)blockIdx.y * hper, h1 = h0 + hper < nhel ? h0 + hper : nhel;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lq = lane >> 4;
   const int64_t ntiles = (n + 15) / 16;
@@ -501,7 +513,7 @@ __global__ void __launch_bounds__(256) k_colour_mfma(const void* jbuf, int64_t n
     // each helicity's colour terms are summed in R, the helicities in FP64 (an FP32 sum
     // over every helicity and colour would lose digits with the number of rows)
     double acc = 0.0;
-    for (int h = 0; h < nhel; ++h) {
+    for (int h = h0; h < h1; ++h) {
       const cx<R>* Jh = J + (int64_t)h * NC * ld;
       R are[KS], aim[KS];
 #pragma unroll
@@ -532,8 +544,24 @@ __global__ void __launch_bounds__(256) k_colour_mfma(const void* jbuf, int64_t n
     // sum the four lane quarters that hold the colours of each event
     acc += __shfl_xor(acc, 16, 64);
     acc += __shfl_xor(acc, 32, 64);
-    if (lq == 0 && ea < n) out[ea] = (accumulate ? out[ea] : 0.0) + acc * scale;
+    if (lq == 0 && ea < n) {
+      if (gridDim.y > 1) reinterpret_cast<double*>(static_cast<cx<R>*>(jbuf) + (int64_t)h0 * NC * ld + tile * 16)[lr] = acc;
+      else out[ea] = (accumulate ? out[ea] : 0.0) + acc * scale;
+    }
   }
+}
+
+// the row ranges' sums of k_colour_mfma, added in order; step: jamps (complex R) from one
+// range's first row to the next one's
+template <class R>
+__global__ void __launch_bounds__(256) k_colour_sum(const void* jbuf, int64_t n, int64_t step, int parts, double scale,
+                                                    int accumulate, double* out) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  const cx<R>* J = static_cast<const cx<R>*>(jbuf) + e / 16 * 16;
+  double acc = 0.0;
+  for (int p = 0; p < parts; ++p) acc += reinterpret_cast<const double*>(J + p * step)[e % 16];
+  out[e] = (accumulate ? out[e] : 0.0) + acc * scale;
 }
 
 // jamps of a single helicity row [NCOLOR][ld] -> (n, NCOLOR, 2) f64
@@ -555,6 +583,9 @@ int64_t ordered_ws_per_row(int precision) {
   return (int64_t)T::NCOLOR * 2 * (precision == 32 ? 4 : 8);
 }
 
+// blocks of k_ordered_jamps per SIMD below which the orderings are split too
+constexpr int ORDERED_WAVES = 2;
+
 // Sub-chunks of events and groups of helicity rows sized to the caller's workspace:
 // the largest helicity group that still leaves a sub-chunk of min(nev, 65536) events
 // (enough waves for every SIMD), then as many events as the workspace holds.
@@ -570,20 +601,18 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
   // whole 16-event tiles per pass: the row stride (n rounded up to 16) then fits too
   int64_t nsub = ws ? ws_bytes / (row * hg) / 16 * 16 : 0;
   if (nsub < 16) return hipErrorInvalidValue;   // the entry point checks the size first
-  // Passes of a whole number of waves per SIMD (4 SIMDs per CU, one event per lane) when a
-  // pass holds few: at one wave per SIMD a pass of 1.07 waves per SIMD takes two wave-times,
-  // with most SIMDs idle in the second.  From 8 waves per SIMD on, the partial last round
-  // costs less than the extra pass that rounding down would add.
+  // passes of equal size, whole 64-event blocks where the workspace allows
+  const int64_t passes = (s.nev + nsub - 1) / nsub;
+  const int64_t even = ((s.nev + passes - 1) / passes + 63) / 64 * 64;
+  if (even < nsub) nsub = even;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  const int64_t fill = (int64_t)cus * 4 * 64;
-  if (nsub > fill && nsub < 8 * fill) nsub = nsub / fill * fill;
   const double scale = 1.0 / (T::CF_DEN * (per_helicity ? 1.0 : T::DENOMINATOR));
   for (int64_t off = 0; off < s.nev; off += nsub) {
     const int64_t n = s.nev - off < nsub ? s.nev - off : nsub;
-    const int64_t tiles = (n + 15) / 16;
+    const int64_t tiles = (n + 15) / 16, blocks = (n + 63) / 64;
     int64_t cblk = (tiles + 3) / 4;
     if (cblk > 65536) cblk = 65536;
     for (int h0 = 0; h0 < nrows; h0 += hg) {
@@ -595,15 +624,36 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
       a.h0 = h0;
       a.nhel = hg;
       a.jbuf = ws;
+      const int ng = ((h0 + hg - 1) >> 2) - (h0 >> 2) + 1;
+      // The orderings are split over blocks while there are fewer blocks than ORDERED_WAVES per
+      // SIMD: a wave's time is then one ordering pair's at least, and what a block computes for
+      // all its orderings (invariants, spinors) is done once more for each range.
+      const int pairs = T::NCOLOR / 2;
+      int64_t parts = (4ll * ORDERED_WAVES * cus + blocks * ng - 1) / (blocks * ng);
+      parts = parts < 1 ? 1 : (parts > pairs ? pairs : parts);
+      const int pper = (int)((pairs + parts - 1) / parts);
+      a.cper = 2 * pper;
+      a.cparts = (pairs + pper - 1) / pper;
+      // ranges of helicity rows of the colour sum: as many as give every SIMD two waves
+      int hper = hg;
+      while (hper > 1 && tiles * (hg / hper) < 8ll * cus) hper /= 2;
+      const int hparts = (hg + hper - 1) / hper;
       const int acc = h0 > 0;
+      const dim3 gj((unsigned)blocks, (unsigned)(ng * a.cparts)), gc((unsigned)cblk, (unsigned)hparts);
+      const int64_t step = (int64_t)hper * T::NCOLOR * a.ld;
+      const dim3 gs((unsigned)((n + 255) / 256));
       if (precision == 32) {
-        hipLaunchKernelGGL((k_ordered_jamps<T, float, 64>), dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, a);
-        hipLaunchKernelGGL((k_colour_mfma<T, float>), dim3((unsigned)cblk), dim3(256), 0, st, (const void*)ws, n, a.ld,
-                           hg, scale, acc, s.out + off);
+        hipLaunchKernelGGL((k_ordered_jamps<T, float, 64>), gj, dim3(64), 0, st, a);
+        hipLaunchKernelGGL((k_colour_mfma<T, float>), gc, dim3(256), 0, st, ws, n, a.ld, hg, hper, scale, acc, s.out + off);
+        if (hparts > 1)
+          hipLaunchKernelGGL((k_colour_sum<float>), gs, dim3(256), 0, st, (const void*)ws, n, step, hparts, scale, acc,
+                             s.out + off);
       } else {
-        hipLaunchKernelGGL((k_ordered_jamps<T, double, 64>), dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, a);
-        hipLaunchKernelGGL((k_colour_mfma<T, double>), dim3((unsigned)cblk), dim3(256), 0, st, (const void*)ws, n,
-                           a.ld, hg, scale, acc, s.out + off);
+        hipLaunchKernelGGL((k_ordered_jamps<T, double, 64>), gj, dim3(64), 0, st, a);
+        hipLaunchKernelGGL((k_colour_mfma<T, double>), gc, dim3(256), 0, st, ws, n, a.ld, hg, hper, scale, acc, s.out + off);
+        if (hparts > 1)
+          hipLaunchKernelGGL((k_colour_sum<double>), gs, dim3(256), 0, st, (const void*)ws, n, step, hparts, scale, acc,
+                             s.out + off);
       }
     }
     if (per_helicity && s.jamp_out) {
