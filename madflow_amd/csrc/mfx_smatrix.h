@@ -42,10 +42,11 @@ __device__ __forceinline__ Params<R> load_params(const SmatrixArgs& a, int64_t e
   return prm;
 }
 
-// sum_ij J_i cf_ij conj(J_j) / den with a real symmetric cf:
+// sum_ij J_i cf_ij conj(J_j) with a real symmetric integer cf (colour_sum: over its
+// denominator):
 //   sum_i cf_ii |J_i|^2 + 2 sum_{i<j} cf_ij Re(J_i conj(J_j))
 template <class T, class R>
-__device__ __forceinline__ R colour_sum(const cx<R> (&J)[T::NCOLOR]) {
+__device__ __forceinline__ R colour_numerator(const cx<R> (&J)[T::NCOLOR]) {
   constexpr int NC = T::NCOLOR;
   R res = R(0);
 #pragma unroll
@@ -60,7 +61,11 @@ __device__ __forceinline__ R colour_sum(const cx<R> (&J)[T::NCOLOR]) {
     }
     res += zr * J[i].re + zi * J[i].im;
   }
-  return res * R(1.0 / T::CF_DEN);
+  return res;
+}
+template <class T, class R>
+__device__ __forceinline__ R colour_sum(const cx<R> (&J)[T::NCOLOR]) {
+  return colour_numerator<T, R>(J) * R(1.0 / T::CF_DEN);
 }
 
 // Per-event invariants inv[k] = 2 k_i.k_j (i < j) of the outgoing momenta k_l = sign_l p_l,
@@ -220,7 +225,7 @@ template <class T> struct ColourLds<T, true> {
   float red[4][64];
 };
 
-// Hot path: all helicity rows for nev events.  The event loop is block-uniform so that
+// All helicity rows for nev events, an event's rows one after another on one lane.  The event loop is block-uniform so that
 // every lane of a wave reaches the wave-wide colour contraction; lanes past the end
 // evaluate the last event again and write nothing.
 template <class T, class R>
@@ -321,6 +326,94 @@ __global__ void __launch_bounds__(256) k_smatrix(SmatrixArgs a) {
   }
 }
 
+// Rows evaluated two at a time by amplitudes2 in k_smatrix_rows, both precisions: the shared
+// currents are a quarter to a half of a row's work.  1e6 events FP64, one row at a time -> two:
+// t t~ 585 -> 352 us, t t~ g 4.52 -> 3.86 ms, u u~ > t t~ 189 -> 126 us, u u~ > t t~ g 968 -> 695 us,
+// u u~ > t t~ g g 15.8 -> 14.0 ms (although it spills 636 B a lane instead of 196).
+template <class T> struct PairedRows {
+  static constexpr bool value = T::MULTI_K == 1;
+};
+
+// Waves per SIMD that k_smatrix_rows is compiled for: two where 256 registers hold a pair of
+// rows, or all but 52 B of it (1e6 events: t t~ g FP32 2,366 -> 1,857 us, u u~ > t t~ g FP64
+// 688 -> 601 us); more colour flows would spill 0.4-1.8 KB a lane (t t~ g FP64 3,854 -> 7,787 us,
+// u u~ > t t~ g g FP32 4,880 -> 5,766 us).
+template <class T, class R> struct RowsWaves {
+  static constexpr int value = T::NCOLOR <= (StableForms<R>::value ? 6 : 4) ? 2 : 1;
+};
+
+// The helicity rows of an event side by side: a block takes E events (a power of two up to 64)
+// and spreads their rows, or pairs of rows, over its 256 lanes, 256 / E at a time.  Each
+// row's colour sum goes to LDS and one lane per event adds the rows in k_smatrix's order, so
+// the FP32 result is the same to the last bit.  A lane that walks every row by itself leaves
+// the chip idle for few events and ends larger calls in a half-empty round: per call, one lane
+// an event -> this kernel, t t~ FP64 16 events 41 -> 17 us (15 of them the host's),
+// u u~ > t t~ g g FP64 30,001 events 1,259 -> 459 us, t t~ g FP32 4,000 events 146 -> 18 us,
+// 500,009 events 1,179 -> 932 us.
+template <class T, class R>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RowsWaves<T, R>::value)))
+k_smatrix_rows(SmatrixArgs a, int64_t ev0, int E) {
+  constexpr bool PAIR = PairedRows<T>::value;
+  constexpr int PER = PAIR ? 2 : 1, NGRP = T::NCOMB / PER;
+  static_assert(NGRP <= 64, "one lane per group of rows");
+  __shared__ R rows[T::NCOMB * 64];
+  __shared__ unsigned short group[64];
+  __shared__ int ngroup;
+  const int t = threadIdx.x;
+  if (t < 64) {                          // the groups of rows that do not vanish, in order
+    unsigned hb = 0u;
+    if (t < NGRP) {
+      if constexpr (PAIR) {
+        constexpr int X = T::MULTI_LEG[0];
+        hb = ((unsigned)t & ((1u << X) - 1u)) | (((unsigned)t >> X) << (X + 1));
+      } else {
+        hb = T::hel_bits(t);
+      }
+    }
+    const bool live = t < NGRP && T::live(hb);
+    const unsigned long long mask = __ballot(live);
+    if (live) group[__popcll(mask & ((1ull << t) - 1ull))] = (unsigned short)hb;
+    if (t == 0) ngroup = __popcll(mask);
+  }
+  __syncthreads();
+  const int ng = ngroup, le = t & (E - 1);
+  const int64_t e0 = ev0 + (int64_t)blockIdx.x * E + le;
+  const int64_t e = e0 < a.nev ? e0 : a.nev - 1;
+  R p[T::NEXTERNAL][4];
+  R inv[T::NINV];
+  load_momenta<T, R>(a.all_ps, e, p);
+  if constexpr (StableForms<R>::value) load_invariants<T, R>(a.all_ps, e, inv);
+  const Params<R> prm = load_params<R>(a, e);
+#pragma unroll 1
+  for (int i = t / E; i < ng; i += 256 / E) {
+#pragma unroll
+    for (int l = 0; l < T::NEXTERNAL; ++l)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) opaque(p[l][k]);
+    if constexpr (StableForms<R>::value) {
+#pragma unroll
+      for (int k = 0; k < T::NINV; ++k) opaque(inv[k]);
+    }
+    const unsigned hb = group[i];
+    cx<R> jamp[T::NCOLOR];
+    if constexpr (PAIR) {
+      cx<R> jamp2[T::NCOLOR];
+      T::template amplitudes2<R>(p, inv, hb, prm, jamp, jamp2);
+      rows[2 * i * E + le] = colour_numerator<T, R>(jamp);
+      rows[(2 * i + 1) * E + le] = colour_numerator<T, R>(jamp2);
+    } else {
+      T::template amplitudes<R>(p, inv, hb, nullptr, prm, jamp);
+      rows[i * E + le] = colour_numerator<T, R>(jamp);
+    }
+  }
+  __syncthreads();
+  if (t < E && e0 < a.nev) {
+    R ans = R(0);
+    for (int i = 0; i < PER * ng; ++i) ans += rows[i * E + t] * R(1.0 / T::CF_DEN);
+    a.out[e0] = double(ans) / T::DENOMINATOR;
+  }
+}
+
 // matrix(all_ps, hel, ...): one explicit helicity vector (may hold 4 = BRST check for a
 // gluon); optionally also returns the jamps.
 template <class T, class R>
@@ -345,6 +438,14 @@ __global__ void __launch_bounds__(256) k_matrix_hel(SmatrixArgs a) {
   }
 }
 
+// Whether large calls run k_smatrix: the processes with 24 colour flows (whose colour sum needs
+// every lane of a wave at once, or whose rows fill the register file by themselves), and
+// FP32 with few groups of rows.
+template <class T, class R> struct KeepsEvents {
+  static constexpr bool value =
+      T::NCOLOR >= 24 || (StableForms<R>::value && T::NCOMB / (T::FILTERED ? 4 : 2) < 16);
+};
+
 struct ProcessEntry {
   const char* name;
   int nexternal, ncomb, ncolor, ndiags, ngraphs;
@@ -356,20 +457,67 @@ struct ProcessEntry {
   int64_t (*ws_per_row)(int precision);
 };
 
+// Which kernel takes a call, and E: k_smatrix_rows (E > 0) or k_smatrix (0).
+// A block of k_smatrix_rows works through ceil(groups E / 256) groups of rows after loading its
+// events (about half a group's time), and a CU takes one such block at a time for the
+// purpose of this estimate, so a smaller E is faster until the blocks outnumber the CUs:
+// u u~ > t t~ g g FP64, 1,000 events: E = 64 259 us, 16 37 us; 30,001 events: 64 522 us, 16 526 us.
+// With few groups of rows the FP32 load (the invariants in FP64) is no longer small beside
+// them, and k_smatrix, which loads an event once, is faster from 1,024 events a CU on:
+// u u~ > t t~ g FP32 200,000 events 110 us against 102 us, 1e6 events 400 us against 475 us.
+// With 16 groups or more it is not (u u~ > t t~ g g 1e6 events 4,934 us against 4,858 us).
+template <class T, class R>
+int events_per_block(int64_t nev) {
+  constexpr int groups = T::NCOMB / (PairedRows<T>::value ? 2 : 1) / (T::FILTERED ? 2 : 1);
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  if (KeepsEvents<T, R>::value && nev > 1024ll * cus) return 0;
+  int best = 64;
+  int64_t least = INT64_MAX;
+  for (int E = 64; E >= 4; E /= 2) {
+    const int64_t blocks = (nev + E - 1) / E;
+    const int64_t cost = (blocks + cus - 1) / cus * (2 * ((groups * E + 255) / 256) + 1);
+    if (cost < least) {
+      least = cost;
+      best = E;
+    }
+  }
+  return best;
+}
+
+template <class T, class R>
+hipError_t launch_smatrix(const SmatrixArgs& a, hipStream_t s) {
+  if constexpr (!MfmaColour<T, R>::value && T::NCOLOR < 24) {
+    const int E = events_per_block<T, R>(a.nev);
+    if (E) {
+      const int64_t most = (int64_t)E << 22;        // events of one launch (its threads fit 32 bits)
+      for (int64_t ev0 = 0; ev0 < a.nev; ev0 += most) {
+        const int64_t n = a.nev - ev0 < most ? a.nev - ev0 : most;
+        hipLaunchKernelGGL((k_smatrix_rows<T, R>), dim3((unsigned)((n + E - 1) / E)), dim3(256), 0, s, a, ev0, E);
+      }
+      return hipGetLastError();
+    }
+  }
+  if constexpr (KeepsEvents<T, R>::value) {
+    int64_t nblk = (a.nev + 255) / 256;
+    if (nblk > (1 << 30)) nblk = 1 << 30;
+    hipLaunchKernelGGL((k_smatrix<T, R>), dim3((unsigned)nblk), dim3(256), 0, s, a);
+  }
+  return hipGetLastError();
+}
+
 template <class T>
 hipError_t launch_process(const SmatrixArgs& a, int precision, int per_helicity, void*, int64_t, hipStream_t s) {
   if (a.nev <= 0) return hipSuccess;
+  if (!per_helicity) return precision == 32 ? launch_smatrix<T, float>(a, s) : launch_smatrix<T, double>(a, s);
   const int block = 256;
   int64_t nblk = (a.nev + block - 1) / block;
   if (nblk > (1 << 30)) nblk = 1 << 30;
   dim3 grid((unsigned)nblk), blk(block);
-  if (precision == 32) {
-    if (per_helicity) hipLaunchKernelGGL((k_matrix_hel<T, float>), grid, blk, 0, s, a);
-    else hipLaunchKernelGGL((k_smatrix<T, float>), grid, blk, 0, s, a);
-  } else {
-    if (per_helicity) hipLaunchKernelGGL((k_matrix_hel<T, double>), grid, blk, 0, s, a);
-    else hipLaunchKernelGGL((k_smatrix<T, double>), grid, blk, 0, s, a);
-  }
+  if (precision == 32) hipLaunchKernelGGL((k_matrix_hel<T, float>), grid, blk, 0, s, a);
+  else hipLaunchKernelGGL((k_matrix_hel<T, double>), grid, blk, 0, s, a);
   return hipGetLastError();
 }
 
