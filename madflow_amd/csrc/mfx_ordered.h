@@ -213,19 +213,44 @@ struct OrderedArgs {
 // Per-lane staging in LDS (lane-major: slot s of lane t at s * BLOCK + t), used as an
 // indexable store: the gluon wavefunctions and the pair invariants are read back in the
 // order of each colour ordering (the ordering index is wave-uniform).
-template <class T, class R>
+template <class T, class R, bool EXPLICIT>
 struct OrderedStage {
   static constexpr int NG = T::NG;
-  static constexpr int NWF = NG * 12;                  // 5 gluons x 6 complex
+  // FP32 runs two waves a SIMD, since one wave alone does not keep its VALU issuing; that takes
+  // at most 256 registers a lane, and at most 80 slots here for 8 waves to fit a CU's 160 KB.
+  // Four gluons (102 slots in full): COMPACT leaves out what is known to be zero, the
+  // polarisations' time component and the imaginary part of their z component (not with an
+  // explicit helicity vector, whose BRST polarisation fills all four real parts), the
+  // fermions' momenta and one number of the anti-top.  Five gluons: the fermions' spinors, 40
+  // slots, go to private memory, read back from cache with a run-time helicity.
+  // t t~ g g, 1,048,576 events: 102 slots (6 waves a CU) 35.2 ms, 82 slots (7) 29.9 ms, 80 slots (8)
+  // 26.8 ms; spinors in private memory 28.7 ms, and three waves a SIMD with them 29.8 ms (272 B of
+  // spills).  t t~ g g g, 50,000 events: one wave a SIMD 33.7 ms, two with 120 slots (5 waves a CU)
+  // 32.2 ms, with 80 slots 26.6 ms although 224 B spill.
+  static constexpr bool COMPACT = !EXPLICIT && NG <= 4;
+  static constexpr int GW = COMPACT ? 9 : 12;
+  static constexpr int NWF = NG * GW;
   // FP32: the pair invariants gluon-gluon and top-gluon (pair_index), then anti-top-gluon
   static constexpr int NPI = StableForms<R>::value ? (NG + 1) * NG / 2 : 0;
   static constexpr int NINV = StableForms<R>::value ? NPI + NG : 0;
-  // FP32: the top and anti-top spinors of both helicities (momentum slots once, spinor
-  // components per helicity), staged once per event; FP64 recomputes them (its LDS
-  // budget is spent)
+  // FP32: the spinor components of the top and the anti-top at both helicities, staged once
+  // per event; FP64 recomputes them (its LDS budget is spent)
   static constexpr int FB = NWF + NINV;
-  static constexpr int NFS = StableForms<R>::value ? 40 : 0;
-  static constexpr int NSLOT = NWF + NINV + NFS;
+  static constexpr int NFM = COMPACT ? 0 : 4;       // momentum slots of a fermion
+  static constexpr int NFS = StableForms<R>::value ? (COMPACT ? 30 : 40) : 0;
+  static constexpr bool PRIVATE = NG > 4;           // the spinors in private memory
+  static constexpr int NSLOT = NWF + NINV + (PRIVATE ? 0 : NFS);
+  // slot of component q (its real part; the imaginary part follows) of the top (anti = 0) or
+  // the anti-top at helicity bit h
+  static constexpr __device__ int fermion(int anti, int h, int q) {
+    return FB + (q < 2 ? 4 * anti + 2 * q
+                       : 2 * NFM + 16 * anti + (COMPACT && anti ? 7 : 8) * h + 2 * (q - 2));
+  }
+  // slot of component q (0, 1: momentum; 2..5: polarisation), part 0 / 1, of a gluon; -1: zero
+  static constexpr __device__ int gluon(int q, int part) {
+    if (!COMPACT || q < 2) return 2 * q + part;
+    return q == 2 ? -1 : (q == 5 ? (part ? -1 : 8) : 4 + 2 * (q - 3) + part);
+  }
 };
 
 // One block takes 64 events through one set of gluon helicities (its four top / anti-top rows)
@@ -236,10 +261,11 @@ struct OrderedStage {
 // wave walking every set of its 64 events: t t~ g g FP64, 1,000 events, 3,117 -> 103 us; t t~ g g g
 // FP32, 257 events, 44.2 -> 0.31 ms, 50,000 events, 42.2 -> 33.7 ms; t t~ g g FP32, 1,048,576
 // events, 37.9 -> 35.2 ms (the momenta no longer stay live across the sets: 244 -> 184 VGPRs).
-template <class T, class R, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) k_ordered_jamps(OrderedArgs a) {
+template <class T, class R, int BLOCK, bool EXPLICIT>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(StableForms<R>::value ? 2 : 1)))
+k_ordered_jamps(OrderedArgs a) {
   constexpr int NG = T::NG, NE = T::NEXTERNAL, NC = T::NCOLOR;
-  using S = OrderedStage<T, R>;
+  using S = OrderedStage<T, R, EXPLICIT>;
   __shared__ R lds[S::NSLOT * BLOCK];
   const int t = threadIdx.x;
   const int64_t el = (int64_t)blockIdx.x * BLOCK + t;
@@ -274,33 +300,74 @@ __global__ void __launch_bounds__(BLOCK) k_ordered_jamps(OrderedArgs a) {
       lds[(S::NWF + S::NPI + x) * BLOCK + t] = R(v);
     }
   }
+  __attribute__((aligned(16))) R spinor[S::PRIVATE ? 40 : 1];
+  R atop_last[2];       // COMPACT: the imaginary part of the anti-top's component 5
   if constexpr (S::NFS > 0) {
-    const int* hv = a.s.use_helv ? a.s.helv : nullptr;
+    const int* hv = EXPLICIT && a.s.use_helv ? a.s.helv : nullptr;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       W<R> top, atop;
       T::template fermions<R>(p, ((unsigned)h << T::TOP_LEG) | ((unsigned)h << T::ATOP_LEG), hv, prm, top, atop);
 #pragma unroll
       for (int q = 0; q < 6; ++q) {
-        const int ot = q < 2 ? 2 * q : 8 + 8 * h + 2 * (q - 2);       // top
-        const int oa = q < 2 ? 4 + 2 * q : 24 + 8 * h + 2 * (q - 2);  // anti-top
-        if (q >= 2 || h == 0) {
-          lds[(S::FB + ot) * BLOCK + t] = top[q].re;
-          lds[(S::FB + ot + 1) * BLOCK + t] = top[q].im;
-          lds[(S::FB + oa) * BLOCK + t] = atop[q].re;
-          lds[(S::FB + oa + 1) * BLOCK + t] = atop[q].im;
+        const int ot = S::fermion(0, h, q), oa = S::fermion(1, h, q);
+        if constexpr (S::PRIVATE) {
+          if (q >= 2 || h == 0) {
+            spinor[ot - S::FB] = top[q].re;
+            spinor[ot + 1 - S::FB] = top[q].im;
+            spinor[oa - S::FB] = atop[q].re;
+            spinor[oa + 1 - S::FB] = atop[q].im;
+          }
+        } else if (q >= 2 || (h == 0 && !S::COMPACT)) {
+          lds[ot * BLOCK + t] = top[q].re;
+          lds[(ot + 1) * BLOCK + t] = top[q].im;
+          lds[oa * BLOCK + t] = atop[q].re;
+          if (!S::COMPACT || q < 5) lds[(oa + 1) * BLOCK + t] = atop[q].im;
+        }
+      }
+      atop_last[h] = atop[5].im;
+    }
+  }
+  // spinor of the top (anti = 0) or anti-top (anti = 1) at helicity bit h, from LDS; COMPACT: the
+  // top's momentum slots from p, the anti-top's, which are not read, left out
+  auto staged_fermion = [&](int anti, int h, W<R>& w) {
+    if constexpr (S::COMPACT) {
+      if (!anti) {
+        w[0] = cx<R>(p[T::TOP_LEG][0], p[T::TOP_LEG][3]);
+        w[1] = cx<R>(p[T::TOP_LEG][1], p[T::TOP_LEG][2]);
+      }
+#pragma unroll
+      for (int q = 2; q < 6; ++q) {
+        const int o = S::fermion(anti, h, q);
+        w[q].re = lds[o * BLOCK + t];
+        if (q < 5 || !anti) {
+          w[q].im = lds[(o + 1) * BLOCK + t];
+        } else {
+          w[q].im = h ? atop_last[1] : atop_last[0];
+          opaque(w[q].im);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        const int o = S::fermion(anti, h, q);
+        if constexpr (S::PRIVATE) {
+          w[q].re = spinor[o - S::FB];
+          w[q].im = spinor[o + 1 - S::FB];
+        } else {
+          w[q].re = lds[o * BLOCK + t];
+          w[q].im = lds[(o + 1) * BLOCK + t];
         }
       }
     }
-  }
-  // spinor of the top (anti = 0) or anti-top (anti = 1) at helicity bit h, from LDS
-  auto staged_fermion = [&](int anti, int h, W<R>& w) {
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-      const int o = q < 2 ? 4 * anti + 2 * q : 8 + 16 * anti + 8 * h + 2 * (q - 2);
-      w[q].re = lds[(S::FB + o) * BLOCK + t];
-      w[q].im = lds[(S::FB + o + 1) * BLOCK + t];
-    }
+  };
+  // one real number of the gluon at slot s; a zero is opaque like a loaded value, so that the
+  // compiler contracts the products it appears in as it does the others
+  auto staged_gluon = [&](int s, int q, int part) -> R {
+    if (S::gluon(q, part) >= 0) return lds[(s * S::GW + S::gluon(q, part)) * BLOCK + t];
+    R z = R(0);
+    opaque(z);
+    return z;
   };
   cx<R>* jb = reinterpret_cast<cx<R>*>(a.jbuf);
   // Helicity rows are enumerated here as r = 4 g + 2 ht + ha: g = the gluon helicities
@@ -329,15 +396,20 @@ __global__ void __launch_bounds__(BLOCK) k_ordered_jamps(OrderedArgs a) {
   unsigned hbg = 0u;
 #pragma unroll
   for (int s = 0; s < NG; ++s) hbg |= ((unsigned)(g >> s) & 1u) << T::gluon_leg(s);
-  const int* helv = a.s.use_helv ? a.s.helv : nullptr;
+  const int* helv = EXPLICIT && a.s.use_helv ? a.s.helv : nullptr;
 #pragma unroll
   for (int s = 0; s < NG; ++s) {
     W<R> gw;
     T::template gluon<R>(p, s, hbg, helv, prm, gw);
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-      lds[(s * 12 + 2 * q) * BLOCK + t] = gw[q].re;
-      lds[(s * 12 + 2 * q + 1) * BLOCK + t] = gw[q].im;
+      if constexpr (S::COMPACT) {
+        if (S::gluon(q, 0) >= 0) lds[(s * S::GW + S::gluon(q, 0)) * BLOCK + t] = gw[q].re;
+        if (S::gluon(q, 1) >= 0) lds[(s * S::GW + S::gluon(q, 1)) * BLOCK + t] = gw[q].im;
+      } else {
+        lds[(s * 12 + 2 * q) * BLOCK + t] = gw[q].re;
+        lds[(s * 12 + 2 * q + 1) * BLOCK + t] = gw[q].im;
+      }
     }
   }
   // Orderings come in lexicographic order, so orderings 2m and 2m+1 share their first
@@ -354,8 +426,13 @@ __global__ void __launch_bounds__(BLOCK) k_ordered_jamps(OrderedArgs a) {
       if (k < PRE && !fresh) continue;
 #pragma unroll
       for (int q = 0; q < 6; ++q) {
-        J[k][k][q].re = lds[(perm[k] * 12 + 2 * q) * BLOCK + t];
-        J[k][k][q].im = lds[(perm[k] * 12 + 2 * q + 1) * BLOCK + t];
+        if constexpr (S::COMPACT) {
+          J[k][k][q].re = staged_gluon(perm[k], q, 0);
+          J[k][k][q].im = staged_gluon(perm[k], q, 1);
+        } else {
+          J[k][k][q].re = lds[(perm[k] * 12 + 2 * q) * BLOCK + t];
+          J[k][k][q].im = lds[(perm[k] * 12 + 2 * q + 1) * BLOCK + t];
+        }
       }
     }
     if constexpr (S::NINV > 0) {
@@ -583,7 +660,10 @@ int64_t ordered_ws_per_row(int precision) {
   return (int64_t)T::NCOLOR * 2 * (precision == 32 ? 4 : 8);
 }
 
-// blocks of k_ordered_jamps per SIMD below which the orderings are split too
+// blocks of k_ordered_jamps per SIMD below which the orderings are split too.  One leaves the
+// second wave of a SIMD out (t t~ g g g FP32, 1,000 events: 1,056 us against 610 us with two); four
+// and eight are within the scatter of the rounds they end in (1,000 events: 652 and 638 us; 2,500
+// events: 1,437 and 1,493 us against 1,711 us; 257 events: 296 and 273 us against 267 us).
 constexpr int ORDERED_WAVES = 2;
 
 // Sub-chunks of events and groups of helicity rows sized to the caller's workspace:
@@ -643,13 +723,15 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
       const int64_t step = (int64_t)hper * T::NCOLOR * a.ld;
       const dim3 gs((unsigned)((n + 255) / 256));
       if (precision == 32) {
-        hipLaunchKernelGGL((k_ordered_jamps<T, float, 64>), gj, dim3(64), 0, st, a);
+        if (T::NG > 4 || s.use_helv) hipLaunchKernelGGL((k_ordered_jamps<T, float, 64, true>), gj, dim3(64), 0, st, a);
+        else hipLaunchKernelGGL((k_ordered_jamps<T, float, 64, false>), gj, dim3(64), 0, st, a);
         hipLaunchKernelGGL((k_colour_mfma<T, float>), gc, dim3(256), 0, st, ws, n, a.ld, hg, hper, scale, acc, s.out + off);
         if (hparts > 1)
           hipLaunchKernelGGL((k_colour_sum<float>), gs, dim3(256), 0, st, (const void*)ws, n, step, hparts, scale, acc,
                              s.out + off);
       } else {
-        hipLaunchKernelGGL((k_ordered_jamps<T, double, 64>), gj, dim3(64), 0, st, a);
+        if (s.use_helv) hipLaunchKernelGGL((k_ordered_jamps<T, double, 64, true>), gj, dim3(64), 0, st, a);
+        else hipLaunchKernelGGL((k_ordered_jamps<T, double, 64, false>), gj, dim3(64), 0, st, a);
         hipLaunchKernelGGL((k_colour_mfma<T, double>), gc, dim3(256), 0, st, ws, n, a.ld, hg, hper, scale, acc, s.out + off);
         if (hparts > 1)
           hipLaunchKernelGGL((k_colour_sum<double>), gs, dim3(256), 0, st, (const void*)ws, n, step, hparts, scale, acc,
