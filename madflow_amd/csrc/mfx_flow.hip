@@ -279,6 +279,13 @@ __device__ __forceinline__ f32x4 mfma_k32(bf16x8 a, bf16x8 b, f32x4 acc) {
   return mfma_bf16(__builtin_shufflevector(a, a, 4, 5, 6, 7), __builtin_shufflevector(b, b, 4, 5, 6, 7), acc);
 }
 
+// LDS ordering between the lanes of one wave
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // first index k of the normalised running sum with cdf[k] >= u
 __device__ __forceinline__ int64_t cdf_search(const double* __restrict__ cdf, int64_t n, double u) {
   int64_t lo = 0, hi = n - 1;          // invariant: the answer lies in [lo, hi]
@@ -516,6 +523,169 @@ k_flow(FlowArgs A, const float* __restrict__ P,
       const int64_t e = s0 + s;
       if (e < A.n) A.x_out[e * D + d] = xs[s * DMAX + d];
     }
+}
+
+// The flow on large batches without saved state: a block of 4 waves takes 64 samples through every
+// layer.  Against k_flow's 16-sample tiles each weight operand fetched from L2 serves four
+// times the samples (42 GB of weights a million samples were most of k_flow's time), and
+// the spline runs on full waves, a sample per lane and a transformed dimension per wave,
+// instead of on one wave of eight.  For that, wave w computes the spline parameters of
+// dimension w, w + 4, ... of all 64 samples itself (four 16-column tiles from the
+// dimension's first column), so that they only pass through its own part of LDS.  Each
+// output element sums the same products in the same order as in k_flow: the results are
+// equal to the last bit.  76 KB of LDS: two blocks on a CU.
+// 1e6 samples of an 8-layer flow, inverse: 8 dimensions 7.14 -> 2.52 ms, 11 dimensions 14.6 -> 3.43 ms,
+// 4 dimensions (6 layers) 4.45 -> 1.63 ms.
+constexpr int WT = 64;          // samples per block
+constexpr int WV = 4;           // waves per block
+constexpr int XP = DMAX + 1;    // row pitch of the coordinates in LDS (a sample per lane)
+
+template <bool INV>
+__global__ void __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(2)))
+k_flow_wide(FlowArgs A, const float* __restrict__ P, const unsigned short* __restrict__ Pb) {
+  const int D = A.geo.D, L = A.geo.L;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int r = lane & 15, kq = (lane >> 4) * 4, k8 = (lane >> 4) * 8;
+  __shared__ float xs[WT * XP], ld_b[WT * XP];
+  __shared__ __attribute__((aligned(16))) float xa[WT * DMAX];
+  __shared__ __attribute__((aligned(16))) unsigned short h2s[WT * WP];
+  // the first hidden layer, then each wave's spline parameters
+  __shared__ __attribute__((aligned(16))) float raws[WV * WT * NPD];
+  unsigned short* h1s = reinterpret_cast<unsigned short*>(raws);
+  static_assert(sizeof(raws) >= sizeof(h2s), "the hidden layer fits the parameters' space");
+  const int64_t s0 = (int64_t)blockIdx.x * WT;
+  for (int q = tid; q < WT * DMAX; q += 64 * WV) {
+    const int s = q / DMAX, d = q % DMAX;
+    xs[s * XP + d] = s0 + s < A.n && d < D ? A.x_in[(s0 + s) * D + d] : 0.5f;
+  }
+  float ldacc = 0.f;                       // of sample tid (tid < WT)
+  for (int step = 0; step < L; ++step) {
+    const int l = INV ? L - 1 - step : step;
+    const LayerGeom& g = A.geo.layer[l];
+    const int nA = g.nA, nB = g.nB, NP = g.NP;
+    const int j1 = tid & (H - 1);
+    bf16x8 w2f[2][H / 32];                 // this wave's column tiles 2 wid and 2 wid + 1
+    float b2[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int n0 = 16 * (2 * wid + u);
+      b2[u] = P[g.ob2 + n0 + r];
+#pragma unroll
+      for (int c = 0; c < H / 32; ++c) w2f[u][c] = ld_bf16x8(Pb + g.oW2t + (n0 + r) * H + 32 * c + k8);
+    }
+    const float b1 = P[g.ob1 + j1];
+    const int ai = g.A[tid % DMAX];
+    __syncthreads();                       // xs holds this layer's input
+#pragma unroll
+    for (int u = 0; u < WT * DMAX / (64 * WV); ++u) {
+      const int q = tid + u * 64 * WV;
+      xa[q] = q % DMAX < nA ? xs[q / DMAX * XP + ai] : 0.f;
+    }
+    __syncthreads();
+    // layer 1 on VALU: thread t computes column t % 128 of half the samples, four inputs at a
+    // time (the inputs past nA are zero, and so are their weights here)
+    {
+      constexpr int NS = WT / 2;
+      const int sb = tid / H * NS;
+      float v[NS];
+#pragma unroll
+      for (int u = 0; u < NS; ++u) v[u] = b1;
+      for (int i0 = 0; i0 < nA; i0 += 4) {
+        float w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = i0 + i < nA ? P[g.oW1 + (i0 + i) * H + j1] : 0.f;
+#pragma unroll
+        for (int u = 0; u < NS; ++u) {
+          const float4 x = *reinterpret_cast<const float4*>(xa + (sb + u) * DMAX + i0);
+          v[u] += x.x * w[0];
+          v[u] += x.y * w[1];
+          v[u] += x.z * w[2];
+          v[u] += x.w * w[3];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NS; ++u) h1s[(sb + u) * WP + j1] = f2bf(fmaxf(v[u], 0.f));
+    }
+    __syncthreads();
+    // layer 2: h2 = relu(h1 W2 + b2)
+    {
+      f32x4 acc[WT / 16][2];
+#pragma unroll
+      for (int m = 0; m < WT / 16; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int K0 = 0; K0 < H; K0 += 32)
+#pragma unroll
+        for (int m = 0; m < WT / 16; ++m) {
+          const bf16x8 a = ld_bf16x8(h1s + (16 * m + r) * WP + K0 + k8);
+          acc[m][0] = mfma_k32(a, w2f[0][K0 / 32], acc[m][0]);
+          acc[m][1] = mfma_k32(a, w2f[1][K0 / 32], acc[m][1]);
+        }
+#pragma unroll
+      for (int m = 0; m < WT / 16; ++m)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            h2s[(16 * m + kq + i) * WP + 16 * (2 * wid + u) + r] = f2bf(fmaxf(acc[m][u][i] + b2[u], 0.f));
+    }
+    __syncthreads();
+    // layer 3 and the spline, a transformed dimension per wave
+    float* raw = raws + wid * WT * NPD;
+    for (int b = wid; b < nB; b += WV) {
+      const int c0 = b * NPD;
+      f32x4 acc[WT / 16][4];
+#pragma unroll
+      for (int m = 0; m < WT / 16; ++m)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[m][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      float b3[4];
+      const unsigned short* w3[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int col = c0 + 16 * u + r < NP ? c0 + 16 * u + r : NP - 1;   // columns past NPD are dropped
+        b3[u] = P[g.ob3 + col];
+        w3[u] = Pb + g.oW3t + col * H + k8;
+      }
+#pragma unroll
+      for (int K0 = 0; K0 < H; K0 += 32) {
+        bf16x8 w[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w[u] = ld_bf16x8(w3[u] + K0);
+#pragma unroll
+        for (int m = 0; m < WT / 16; ++m) {
+          const bf16x8 a = ld_bf16x8(h2s + (16 * m + r) * WP + K0 + k8);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) acc[m][u] = mfma_k32(a, w[u], acc[m][u]);
+        }
+      }
+      wave_sync();                         // this wave's previous dimension is read
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (16 * u + r < NPD) {
+#pragma unroll
+          for (int m = 0; m < WT / 16; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) raw[(16 * m + kq + i) * NPD + 16 * u + r] = acc[m][u][i] + b3[u];
+        }
+      wave_sync();
+      const int d = g.B[b];
+      const float x = xs[lane * XP + d];
+      const SplineEval sp = INV ? rq_inverse(raw + lane * NPD, x) : rq_forward(raw + lane * NPD, x);
+      xs[lane * XP + d] = sp.z;
+      ld_b[lane * XP + b] = sp.ld;
+    }
+    __syncthreads();
+    if (tid < WT) {
+      float ld = 0.f;
+      for (int b = 0; b < nB; ++b) ld += ld_b[tid * XP + b];
+      ldacc += ld;
+    }
+  }
+  if (tid < WT && s0 + tid < A.n) A.logdet[s0 + tid] = ldacc;
+  for (int q = tid; q < WT * D; q += 64 * WV) {
+    const int s = q / D, d = q % D;
+    if (s0 + s < A.n) A.x_out[(s0 + s) * D + d] = xs[s * XP + d];
+  }
 }
 
 // ------------------------------------------------------------------ backward
@@ -1314,7 +1484,25 @@ static int nb_bound(const FlowGeom& G) {
   return m <= 4 ? 4 : (m <= 8 ? 8 : 16);
 }
 
+// Samples that k_flow's blocks hold at once (two tiles on a CU at up to 4 transformed
+// dimensions, else one): up to there its eight waves a tile end sooner, beyond it needs a second
+// round and k_flow_wide takes over.  8-dim flow, 8,192 samples: k_flow 65 us, k_flow_wide 72 us;
+// 16,384 samples: 125 us, 75 us.  11-dim flow, 4,000 samples: 69 us, 97 us; 8,192: 128 us, 97 us.
+static int64_t flow_round(const FlowGeom& G) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  return (int64_t)cus * TILE * (nb_bound(G) <= 4 ? 2 : 1);
+}
+
 static void launch_flow(const FlowArgs& A, hipStream_t s, const float* P, const unsigned short* Pb) {
+  if (!A.save && !A.cdf && A.n > flow_round(A.geo)) {
+    const dim3 gw((unsigned)((A.n + WT - 1) / WT));
+    if (A.inverse) hipLaunchKernelGGL(k_flow_wide<true>, gw, dim3(64 * WV), 0, s, A, P, Pb);
+    else hipLaunchKernelGGL(k_flow_wide<false>, gw, dim3(64 * WV), 0, s, A, P, Pb);
+    return;
+  }
   const dim3 grid((unsigned)ntiles_of(A.n));
   switch (nb_bound(A.geo)) {
     case 4: hipLaunchKernelGGL(k_flow<4>, grid, dim3(NT), 0, s, A, P, Pb); break;
