@@ -19,9 +19,9 @@
 // fermion-flow factor of the generated jamps.  Summed over the Feynman diagrams
 // consistent with an ordering, these give exactly the jamp of that ordering.
 //
-// Kernel 1 (k_ordered_jamps): one event per lane, every helicity row, every ordering;
-// each finished jamp is stored to a workspace [helicity][colour][event] (coalesced),
-// so no lane ever holds more than one ordering's currents.
+// Kernel 1 (k_ordered_jamps in FP32, k_ordered_mirror in FP64): one event per lane; each
+// finished jamp is stored to a workspace [helicity][colour][event] (coalesced), so no lane
+// ever holds more than one ordering's currents.
 // Kernel 2 (k_colour_mfma): |M|^2 = sum_h Re(J_h^dagger CF J_h) / (CF_DEN * DENOMINATOR)
 // as a batched dense contraction on the matrix cores: per helicity, the integer colour
 // matrix (NCOLOR x NCOLOR) times a 16-event tile of Re J and Im J (NCOLOR x 16) with
@@ -160,7 +160,6 @@ __device__ __forceinline__ void ordered_ranges(W<R> (&J)[NG][NG], cx<R> (&S)[NG]
 template <int NG, int O0, int O1, class R>
 __device__ __forceinline__ void ordered_top_line(W<R> (&O)[NG], const W<R> (&J)[NG][NG], const R (&rt)[NG],
                                                  const Params<R>& prm) {
-  constexpr bool INV = StableForms<R>::value;
 #pragma unroll
   for (int j = O0; j <= O1; ++j) {
     VslashF<R> x = vslash_f(O[0], J[0][j - 1]);
@@ -170,13 +169,7 @@ __device__ __forceinline__ void ordered_top_line(W<R> (&O)[NG], const W<R> (&J)[
     O[j][1] = O[0][1] + J[0][j - 1][1];
     R P[4];
     mom_out(O[j], P);
-    R den2;
-    if constexpr (INV) {
-      den2 = rt[j];
-    } else {
-      den2 = den_from_slots(P, prm.mdl_MT);
-    }
-    ffv1_1_col(x, prm.GC_11, prm.mdl_MT, prm.mdl_WT, den2, P, O[j]);
+    ffv1_1_col(x, prm.GC_11, prm.mdl_MT, prm.mdl_WT, rt[j], P, O[j]);
   }
 }
 
@@ -195,6 +188,87 @@ __device__ __forceinline__ cx<R> ordered_jamp(const W<R>& atop, const VslashF<R>
   return -ffv1_0_col(atop, x, prm.GC_11);
 }
 
+// The top line and closing column of a word (REV = false) or of its reversal, from the word's
+// currents: a colour-ordered gluon current of m letters is (-1)^(m + 1) times that of the
+// letters reversed (Berends and Giele, as above).  The momentum slots of currents of two or
+// more letters are not read.
+template <class R> __device__ __forceinline__ void sub_col(VslashF<R>& acc, const VslashF<R>& x) {
+  acc.c2 -= x.c2;
+  acc.c3 -= x.c3;
+  acc.c4 -= x.c4;
+  acc.c5 -= x.c5;
+}
+// sum over i of gamma.J(i..last) O(i)
+template <bool REV, int NG, class R>
+__device__ __forceinline__ VslashF<R> word_col(const W<R> (&O)[NG], const W<R> (&J)[NG][NG], int last) {
+  VslashF<R> x = vslash_f(O[last], REV ? J[NG - 1 - last][NG - 1 - last] : J[last][last]);
+#pragma unroll
+  for (int i = 0; i < last; ++i) {
+    const VslashF<R> t = vslash_f(O[i], REV ? J[NG - 1 - last][NG - 1 - i] : J[i][last]);
+    if (REV && (last - i) % 2) sub_col(x, t);
+    else add_col(x, t);
+  }
+  return x;
+}
+// O(1..NG-1), then the closing column
+template <bool REV, int NG, class R>
+__device__ __forceinline__ VslashF<R> word_top_line(W<R> (&O)[NG], const W<R> (&J)[NG][NG], const Params<R>& prm) {
+#pragma unroll
+  for (int j = 1; j < NG; ++j) {
+    const VslashF<R> x = word_col<REV>(O, J, j - 1);
+    const int k = REV ? NG - j : j - 1;
+    O[j][0] = O[j - 1][0] + J[k][k][0];
+    O[j][1] = O[j - 1][1] + J[k][k][1];
+    R P[4];
+    mom_out(O[j], P);
+    ffv1_1_col(x, prm.GC_11, prm.mdl_MT, prm.mdl_WT, den_from_slots(P, prm.mdl_MT), P, O[j]);
+  }
+  return word_col<REV>(O, J, NG - 1);
+}
+
+// The walk of the FP64 kernel: NC / 2 words in cycles of rotations.  Cycle m starts with the m-th
+// permutation (in lexicographic order) whose first letter is 0 and whose second is below its
+// last; the next word moves the first letter to the end.  The words and their reversals are
+// all orderings.  at[c] and rev[c]: the colour rows (lexicographic numbers) of word c and of
+// its reversal.
+template <int NG, int NC>
+struct MirrorWalk {
+  unsigned char at[NC / 2], rev[NC / 2];
+};
+template <int NG, int NC>
+constexpr MirrorWalk<NG, NC> mirror_walk() {
+  MirrorWalk<NG, NC> t{};
+  int n = 0;
+  for (int m = 0; m < NC / NG; ++m) {                 // permutations with first letter 0
+    int w[NG] = {}, used[NG] = {}, rem = m, fact = NC / NG;
+    used[0] = 1;
+    for (int k = 1; k < NG; ++k) {                    // digits of m in the factorial base
+      fact /= NG - k;
+      int d = rem / fact, x = 1;
+      rem %= fact;
+      while (used[x] || d-- > 0) ++x;
+      w[k] = x;
+      used[x] = 1;
+    }
+    if (w[1] > w[NG - 1]) continue;
+    for (int r = 0; r < NG; ++r, ++n)
+      for (int way = 0; way < 2; ++way) {
+        int rank = 0, f = NC;
+        for (int k = 0; k < NG; ++k) {
+          const int a = w[(r + (way ? NG - 1 - k : k)) % NG];
+          int less = 0;
+          for (int l = k + 1; l < NG; ++l) less += w[(r + (way ? NG - 1 - l : l)) % NG] < a;
+          f /= NG - k;
+          rank += less * f;
+        }
+        (way ? t.rev : t.at)[n] = (unsigned char)rank;
+      }
+  }
+  return t;
+}
+template <int NG, int NC>
+__constant__ constexpr MirrorWalk<NG, NC> MIRROR_WALK = mirror_walk<NG, NC>();
+
 // the top-line currents O(1..N-1) of both top helicities (empty when unused)
 template <class R, int N, bool ON> struct TopPrefix { W<R> o[2][N]; };
 template <class R, int N> struct TopPrefix<R, N, false> {};
@@ -210,10 +284,10 @@ struct OrderedArgs {
   void* jbuf;           // [nhel][NCOLOR][n] complex R
 };
 
-// Per-lane staging in LDS (lane-major: slot s of lane t at s * BLOCK + t), used as an
+// Per-lane staging of the FP32 kernel in LDS (lane-major: slot s of lane t at s * BLOCK + t), an
 // indexable store: the gluon wavefunctions and the pair invariants are read back in the
 // order of each colour ordering (the ordering index is wave-uniform).
-template <class T, class R, bool EXPLICIT>
+template <class T, bool EXPLICIT>
 struct OrderedStage {
   static constexpr int NG = T::NG;
   // FP32 runs two waves a SIMD, since one wave alone does not keep its VALU issuing; that takes
@@ -230,14 +304,12 @@ struct OrderedStage {
   static constexpr bool COMPACT = !EXPLICIT && NG <= 4;
   static constexpr int GW = COMPACT ? 9 : 12;
   static constexpr int NWF = NG * GW;
-  // FP32: the pair invariants gluon-gluon and top-gluon (pair_index), then anti-top-gluon
-  static constexpr int NPI = StableForms<R>::value ? (NG + 1) * NG / 2 : 0;
-  static constexpr int NINV = StableForms<R>::value ? NPI + NG : 0;
-  // FP32: the spinor components of the top and the anti-top at both helicities, staged once
-  // per event; FP64 recomputes them (its LDS budget is spent)
+  // the pair invariants gluon-gluon and top-gluon (pair_index), then anti-top-gluon
+  static constexpr int NPI = (NG + 1) * NG / 2, NINV = NPI + NG;
+  // the spinor components of the top and the anti-top at both helicities, staged once per event
   static constexpr int FB = NWF + NINV;
   static constexpr int NFM = COMPACT ? 0 : 4;       // momentum slots of a fermion
-  static constexpr int NFS = StableForms<R>::value ? (COMPACT ? 30 : 40) : 0;
+  static constexpr int NFS = COMPACT ? 30 : 40;
   static constexpr bool PRIVATE = NG > 4;           // the spinors in private memory
   static constexpr int NSLOT = NWF + NINV + (PRIVATE ? 0 : NFS);
   // slot of component q (its real part; the imaginary part follows) of the top (anti = 0) or
@@ -261,11 +333,11 @@ struct OrderedStage {
 // wave walking every set of its 64 events: t t~ g g FP64, 1,000 events, 3,117 -> 103 us; t t~ g g g
 // FP32, 257 events, 44.2 -> 0.31 ms, 50,000 events, 42.2 -> 33.7 ms; t t~ g g FP32, 1,048,576
 // events, 37.9 -> 35.2 ms (the momenta no longer stay live across the sets: 244 -> 184 VGPRs).
-template <class T, class R, int BLOCK, bool EXPLICIT>
-__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(StableForms<R>::value ? 2 : 1)))
-k_ordered_jamps(OrderedArgs a) {
+template <class T, int BLOCK, bool EXPLICIT>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) k_ordered_jamps(OrderedArgs a) {
+  typedef float R;
   constexpr int NG = T::NG, NE = T::NEXTERNAL, NC = T::NCOLOR;
-  using S = OrderedStage<T, R, EXPLICIT>;
+  using S = OrderedStage<T, EXPLICIT>;
   __shared__ R lds[S::NSLOT * BLOCK];
   const int t = threadIdx.x;
   const int64_t el = (int64_t)blockIdx.x * BLOCK + t;
@@ -274,7 +346,7 @@ k_ordered_jamps(OrderedArgs a) {
   R p[NE][4];
   load_momenta<T, R>(a.s.all_ps, e, p);
   const Params<R> prm = load_params<R>(a.s, e);
-  if constexpr (S::NINV > 0) {
+  {
     // 2 k_x.k_y in FP64 for x, y among (gluon slots 0..NG-1, top = slot NG)
     const double* src = a.s.all_ps + e * (NE * 4);
     double k[NG + 1][4];
@@ -302,7 +374,7 @@ k_ordered_jamps(OrderedArgs a) {
   }
   __attribute__((aligned(16))) R spinor[S::PRIVATE ? 40 : 1];
   R atop_last[2];       // COMPACT: the imaginary part of the anti-top's component 5
-  if constexpr (S::NFS > 0) {
+  {
     const int* hv = EXPLICIT && a.s.use_helv ? a.s.helv : nullptr;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -384,12 +456,12 @@ k_ordered_jamps(OrderedArgs a) {
   constexpr int PRE = NG - 2;
   W<R> J[NG][NG], O[NG];
   cx<R> SD[NG][NG];   // adjacent-range dot sums S(a..b) of the four-gluon terms
-  // FP32, five or more gluons: the top-line currents O(1..PRE) of both top helicities,
-  // kept from the first ordering of a pair for the second.  Not for FP64 (no registers
-  // to spare) nor for four gluons (the kernel fits two waves per SIMD without them).
-  constexpr bool SHARE_TOP = S::NFS > 0 && NG >= 5;
+  // Five or more gluons: the top-line currents O(1..PRE) of both top helicities, kept from
+  // the first ordering of a pair for the second (for four gluons they would cost the second
+  // wave per SIMD).
+  constexpr bool SHARE_TOP = NG >= 5;
   TopPrefix<R, PRE + 1, SHARE_TOP> OP;
-  // FP32 forms: the word's pair invariants (gluon-gluon pp, top-gluon tp, anti-top-gluon
+  // The word's pair invariants (gluon-gluon pp, top-gluon tp, anti-top-gluon
   // ap) and the top-line denominators rt (above); pp of the prefix pairs carries over to
   // the second ordering of a pair
   R pp[NG][NG], tp[NG], ap[NG], rt[NG];
@@ -435,7 +507,7 @@ k_ordered_jamps(OrderedArgs a) {
         }
       }
     }
-    if constexpr (S::NINV > 0) {
+    {
       // the word's pair invariants (the prefix pairs of a pair's second ordering are the
       // first's), and rt[j] for the top with the first j gluons from the shorter of its
       // two forms
@@ -486,8 +558,7 @@ k_ordered_jamps(OrderedArgs a) {
         const int rb = 4 * g + 2 * ht;
         if (rb + 1 < r0 || rb >= r1) continue;
         W<R> top, atop;
-        if constexpr (S::NFS > 0) staged_fermion(0, ht, top);
-        else T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG), helv, prm, top, atop);
+        staged_fermion(0, ht, top);
         O[0] = top;
         // O(1..PRE) only involve the prefix gluons: computed once per pair of orderings
         if (fresh) {
@@ -504,9 +575,7 @@ k_ordered_jamps(OrderedArgs a) {
         for (int ha = 0; ha < 2; ++ha) {
           const int r = rb + ha;
           if (r < r0 || r >= r1) continue;
-          if constexpr (S::NFS > 0) staged_fermion(1, ha, atop);
-          else if (ha) T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG) | (1u << T::ATOP_LEG), helv,
-                                               prm, top, atop);
+          staged_fermion(1, ha, atop);
           jb[((int64_t)(r - r0) * NC + c) * a.ld + el] = ordered_jamp(atop, x, prm);
         }
       }
@@ -516,8 +585,7 @@ k_ordered_jamps(OrderedArgs a) {
         const int rb = 4 * g + 2 * ht;
         if (rb + 1 < r0 || rb >= r1) continue;
         W<R> top, atop;
-        if constexpr (S::NFS > 0) staged_fermion(0, ht, top);
-        else T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG), helv, prm, top, atop);
+        staged_fermion(0, ht, top);
         O[0] = top;
         ordered_top_line<NG, 1, NG - 1, R>(O, J, rt, prm);
         const VslashF<R> x = ordered_close_col<NG, R>(O, J);
@@ -525,11 +593,145 @@ k_ordered_jamps(OrderedArgs a) {
         for (int ha = 0; ha < 2; ++ha) {
           const int r = rb + ha;
           if (r < r0 || r >= r1) continue;
-          if constexpr (S::NFS > 0) staged_fermion(1, ha, atop);
-          else if (ha) T::template fermions<R>(p, hbg | ((unsigned)ht << T::TOP_LEG) | (1u << T::ATOP_LEG), helv,
-                                               prm, top, atop);
+          staged_fermion(1, ha, atop);
           jb[((int64_t)(r - r0) * NC + c) * a.ld + el] = ordered_jamp(atop, x, prm);
         }
+      }
+    }
+  }
+}
+
+// The FP64 kernel: blocks as k_ordered_jamps, but each word is evaluated together with its
+// reversal, and the words come in cycles of rotations (MirrorWalk): the next word keeps every
+// current but those that end in its new last letter, so one current of each length is
+// computed for two orderings.  (FP32 keeps the currents of each ordering apart: a current's last
+// bits depend on where in the word the compiler contracts it, and FP32 results are held to
+// them.)  30,001 events, against every ordering by itself: t t~ g g 1,580 -> 998 us, t t~ g g g 45.9
+// -> 42.0 ms (its currents do not fit 512 registers: 1.4 KB of spills a lane).  Momenta of ranges
+// are added up again for each word; carried along they made t t~ g g spill and take 1,152 us.
+// LDS: the gluons, then the spinor components of the top and the anti-top at both helicities;
+// one wave per SIMD (the currents fill the registers), so four blocks a CU may take 40 KB each.
+template <class T, bool EXPLICIT>
+struct MirrorStage {
+  static constexpr int NG = T::NG;
+  // a polarisation's time component and the imaginary part of its z component are zero, except
+  // with an explicit helicity vector (BRST)
+  static constexpr int GW = EXPLICIT ? 12 : 9;
+  static constexpr int FB = NG * GW, NSLOT = FB + 32;
+  static constexpr __device__ int gluon(int q, int part) {
+    if (EXPLICIT || q < 2) return 2 * q + part;
+    return q == 2 ? -1 : (q == 5 ? (part ? -1 : 8) : 4 + 2 * (q - 3) + part);
+  }
+};
+
+template <class T, int BLOCK, bool EXPLICIT>
+__global__ void __launch_bounds__(BLOCK) k_ordered_mirror(OrderedArgs a) {
+  typedef double R;
+  constexpr int NG = T::NG, NE = T::NEXTERNAL, NC = T::NCOLOR, NW = NC / 2;
+  using S = MirrorStage<T, EXPLICIT>;
+  __shared__ R lds[S::NSLOT * BLOCK];
+  const int t = threadIdx.x;
+  const int64_t el = (int64_t)blockIdx.x * BLOCK + t;
+  if (el >= a.n) return;                 // no block-level synchronisation below
+  const int64_t e = a.ev0 + el;
+  R p[NE][4];
+  load_momenta<T, R>(a.s.all_ps, e, p);
+  const Params<R> prm = load_params<R>(a.s, e);
+  const int* helv = EXPLICIT ? a.s.helv : nullptr;
+  const int r0 = a.h0, r1 = a.h0 + a.nhel;
+  const int g = (r0 >> 2) + (int)blockIdx.y / a.cparts;
+  const int c0 = ((int)blockIdx.y % a.cparts) * a.cper, c1 = c0 + a.cper < NW ? c0 + a.cper : NW;
+  unsigned hbg = 0u;
+#pragma unroll
+  for (int s = 0; s < NG; ++s) hbg |= ((unsigned)(g >> s) & 1u) << T::gluon_leg(s);
+#pragma unroll
+  for (int s = 0; s < NG; ++s) {
+    W<R> gw;
+    T::template gluon<R>(p, s, hbg, helv, prm, gw);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      if (S::gluon(q, 0) >= 0) lds[(s * S::GW + S::gluon(q, 0)) * BLOCK + t] = gw[q].re;
+      if (S::gluon(q, 1) >= 0) lds[(s * S::GW + S::gluon(q, 1)) * BLOCK + t] = gw[q].im;
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    W<R> top, atop;
+    T::template fermions<R>(p, ((unsigned)h << T::TOP_LEG) | ((unsigned)h << T::ATOP_LEG), helv, prm, top, atop);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int o = S::FB + 8 * h + 2 * q;
+      lds[o * BLOCK + t] = top[q + 2].re;
+      lds[(o + 1) * BLOCK + t] = top[q + 2].im;
+      lds[(o + 16) * BLOCK + t] = atop[q + 2].re;
+      lds[(o + 17) * BLOCK + t] = atop[q + 2].im;
+    }
+  }
+  // spinor components of the top (anti = 0) or anti-top (anti = 1) at helicity bit h
+  auto spinor = [&](int anti, int h, W<R>& w) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int o = S::FB + 16 * anti + 8 * h + 2 * q;
+      w[q + 2] = cx<R>(lds[o * BLOCK + t], lds[(o + 1) * BLOCK + t]);
+    }
+  };
+  cx<R>* jb = reinterpret_cast<cx<R>*>(a.jbuf);
+  W<R> J[NG][NG], O[NG];
+  cx<R> SD[NG][NG];
+  R pp[NG][NG];           // FP32's invariants, not read here
+#pragma unroll 1
+  for (int c = c0; c < c1; ++c) {
+    const int row = MIRROR_WALK<NG, NC>.at[c], rrow = MIRROR_WALK<NG, NC>.rev[c];
+    if (c == c0 || c % NG == 0) {
+#pragma unroll
+      for (int k = 0; k < NG; ++k) {
+        const int s = T::perm(row, k);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+          J[k][k][q].re = S::gluon(q, 0) >= 0 ? lds[(s * S::GW + S::gluon(q, 0)) * BLOCK + t] : R(0);
+          J[k][k][q].im = S::gluon(q, 1) >= 0 ? lds[(s * S::GW + S::gluon(q, 1)) * BLOCK + t] : R(0);
+        }
+      }
+      ordered_ranges<NG, 1, NG - 1, R>(J, SD, pp, prm);
+    } else {
+      const W<R> first = J[0][0];
+#pragma unroll
+      for (int x = 0; x < NG - 1; ++x) J[x][x] = J[x + 1][x + 1];
+#pragma unroll
+      for (int x = 0; x < NG - 1; ++x) {
+#pragma unroll
+        for (int y = x + 1; y < NG - 1; ++y) {
+#pragma unroll
+          for (int q = 2; q < 6; ++q) J[x][y][q] = J[x + 1][y + 1][q];
+          SD[x][y] = SD[x + 1][y + 1];
+          // momenta are added up again rather than carried in registers
+          J[x][y][0] = J[x][y - 1][0] + J[y][y][0];
+          J[x][y][1] = J[x][y - 1][1] + J[y][y][1];
+        }
+      }
+      J[NG - 1][NG - 1] = first;
+    }
+    ordered_ranges<NG, NG - 1, NG, R>(J, SD, pp, prm);
+#pragma unroll 1
+    for (int ht = 0; ht < 2; ++ht) {
+      const int rb = 4 * g + 2 * ht;
+      if (rb + 1 < r0 || rb >= r1) continue;
+      __builtin_amdgcn_sched_barrier(0);
+      O[0][0] = cx<R>(p[T::TOP_LEG][0], p[T::TOP_LEG][3]);
+      O[0][1] = cx<R>(p[T::TOP_LEG][1], p[T::TOP_LEG][2]);
+      spinor(0, ht, O[0]);
+      const VslashF<R> x = word_top_line<false, NG, R>(O, J, prm);
+      __builtin_amdgcn_sched_barrier(0);
+      const VslashF<R> xr = word_top_line<true, NG, R>(O, J, prm);
+#pragma unroll 1
+      for (int ha = 0; ha < 2; ++ha) {
+        const int r = rb + ha;
+        if (r < r0 || r >= r1) continue;
+        W<R> atop;
+        spinor(1, ha, atop);
+        cx<R>* out = jb + (int64_t)(r - r0) * NC * a.ld + el;
+        out[row * a.ld] = ordered_jamp(atop, x, prm);
+        out[rrow * a.ld] = ordered_jamp(atop, xr, prm);
       }
     }
   }
@@ -705,15 +907,17 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
       a.nhel = hg;
       a.jbuf = ws;
       const int ng = ((h0 + hg - 1) >> 2) - (h0 >> 2) + 1;
-      // The orderings are split over blocks while there are fewer blocks than ORDERED_WAVES per
-      // SIMD: a wave's time is then one ordering pair's at least, and what a block computes for
-      // all its orderings (invariants, spinors) is done once more for each range.
-      const int pairs = T::NCOLOR / 2;
+      // The orderings (FP64: words, for two orderings each) are split over blocks while there are
+      // fewer blocks than ORDERED_WAVES per SIMD.  What a block computes for all of them
+      // (invariants, spinors) is done once more for each range, and a range starts its first
+      // word afresh: FP32 ranges are whole pairs, longer FP64 ranges whole cycles.
+      const int unit = precision == 32 ? 2 : 1, count = T::NCOLOR / 2;
       int64_t parts = (4ll * ORDERED_WAVES * cus + blocks * ng - 1) / (blocks * ng);
-      parts = parts < 1 ? 1 : (parts > pairs ? pairs : parts);
-      const int pper = (int)((pairs + parts - 1) / parts);
-      a.cper = 2 * pper;
-      a.cparts = (pairs + pper - 1) / pper;
+      parts = parts < 1 ? 1 : (parts > count ? count : parts);
+      a.cper = (int)((count + parts - 1) / parts);
+      if (precision == 64 && a.cper > T::NG) a.cper = (a.cper + T::NG - 1) / T::NG * T::NG;
+      a.cparts = (count + a.cper - 1) / a.cper;
+      a.cper *= unit;
       // ranges of helicity rows of the colour sum: as many as give every SIMD two waves
       int hper = hg;
       while (hper > 1 && tiles * (hg / hper) < 8ll * cus) hper /= 2;
@@ -723,15 +927,15 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
       const int64_t step = (int64_t)hper * T::NCOLOR * a.ld;
       const dim3 gs((unsigned)((n + 255) / 256));
       if (precision == 32) {
-        if (T::NG > 4 || s.use_helv) hipLaunchKernelGGL((k_ordered_jamps<T, float, 64, true>), gj, dim3(64), 0, st, a);
-        else hipLaunchKernelGGL((k_ordered_jamps<T, float, 64, false>), gj, dim3(64), 0, st, a);
+        if (T::NG > 4 || s.use_helv) hipLaunchKernelGGL((k_ordered_jamps<T, 64, true>), gj, dim3(64), 0, st, a);
+        else hipLaunchKernelGGL((k_ordered_jamps<T, 64, false>), gj, dim3(64), 0, st, a);
         hipLaunchKernelGGL((k_colour_mfma<T, float>), gc, dim3(256), 0, st, ws, n, a.ld, hg, hper, scale, acc, s.out + off);
         if (hparts > 1)
           hipLaunchKernelGGL((k_colour_sum<float>), gs, dim3(256), 0, st, (const void*)ws, n, step, hparts, scale, acc,
                              s.out + off);
       } else {
-        if (s.use_helv) hipLaunchKernelGGL((k_ordered_jamps<T, double, 64, true>), gj, dim3(64), 0, st, a);
-        else hipLaunchKernelGGL((k_ordered_jamps<T, double, 64, false>), gj, dim3(64), 0, st, a);
+        if (s.use_helv) hipLaunchKernelGGL((k_ordered_mirror<T, 64, true>), gj, dim3(64), 0, st, a);
+        else hipLaunchKernelGGL((k_ordered_mirror<T, 64, false>), gj, dim3(64), 0, st, a);
         hipLaunchKernelGGL((k_colour_mfma<T, double>), gc, dim3(256), 0, st, ws, n, a.ld, hg, hper, scale, acc, s.out + off);
         if (hparts > 1)
           hipLaunchKernelGGL((k_colour_sum<double>), gs, dim3(256), 0, st, (const void*)ws, n, step, hparts, scale, acc,
