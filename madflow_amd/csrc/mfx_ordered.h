@@ -753,8 +753,8 @@ template <class R> struct Vec4;
 template <> struct Vec4<float> { typedef mfx_f32x4 type; };
 template <> struct Vec4<double> { typedef mfx_f64x4 type; };
 
-// |M|^2 of the events of one sub-chunk from their jamps: one wave per 16-event tile and range
-// of hper helicity rows (blockIdx.y), four tiles per block.  Per helicity and tile the matrix cores form D = CF J^T
+// |M|^2 of the events of one sub-chunk from their jamps: one wave per item, a 16-event tile and a
+// range of hper helicity rows, the waves taking items in turn.  Per helicity and tile the matrix cores form D = CF J^T
 // (NCP x 16: colour rows, event columns) from the integer colour matrix (A operand, in
 // LDS) and the tile's jamps (B operand: lane (i, q) holds J[event i][colour 4 s + q] for
 // every k-step s), then each lane dots its D entries with jamps it already holds.  For
@@ -793,11 +793,13 @@ __global__ void __launch_bounds__(256) k_colour_mfma(void* jbuf, int64_t n, int6
   }
   __syncthreads();
   const cx<R>* J = reinterpret_cast<const cx<R>*>(jbuf);
-  const int h0 = (int)blockIdx.y * hper, h1 = h0 + hper < nhel ? h0 + hper : nhel;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 15, lq = lane >> 4;
-  const int64_t ntiles = (n + 15) / 16;
-  for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < ntiles; tile += (int64_t)gridDim.x * 4) {
+  // 32 bits hold the items: the jamps of 2^31 of them would take terabytes
+  const unsigned ntiles = (unsigned)((n + 15) / 16), parts = (unsigned)((nhel + hper - 1) / hper);
+  for (unsigned item = blockIdx.x * 4 + wave; item < ntiles * parts; item += gridDim.x * 4) {
+    const int64_t tile = item % ntiles;
+    const int h0 = (int)(item / ntiles) * hper, h1 = h0 + hper < nhel ? h0 + hper : nhel;
     const int64_t ea = tile * 16 + lr;          // the event of this lane's B column
     // each helicity's colour terms are summed in R, the helicities in FP64 (an FP32 sum
     // over every helicity and colour would lose digits with the number of rows)
@@ -834,7 +836,7 @@ __global__ void __launch_bounds__(256) k_colour_mfma(void* jbuf, int64_t n, int6
     acc += __shfl_xor(acc, 16, 64);
     acc += __shfl_xor(acc, 32, 64);
     if (lq == 0 && ea < n) {
-      if (gridDim.y > 1) reinterpret_cast<double*>(static_cast<cx<R>*>(jbuf) + (int64_t)h0 * NC * ld + tile * 16)[lr] = acc;
+      if (parts > 1) reinterpret_cast<double*>(static_cast<cx<R>*>(jbuf) + (int64_t)h0 * NC * ld + tile * 16)[lr] = acc;
       else out[ea] = (accumulate ? out[ea] : 0.0) + acc * scale;
     }
   }
@@ -883,6 +885,10 @@ int64_t ordered_ws_per_row(int precision) {
 // events: 1,437 and 1,493 us against 1,711 us; 257 events: 296 and 273 us against 267 us).
 constexpr int ORDERED_WAVES = 2;
 
+// (tile, rows) items per wave slot of k_colour_mfma: t t~ g g g FP32, 50,000 events, 27.2 ms a call
+// with one round of tiles, 26.0 ms with 4 and with 8 (the colour sum 4.05 -> 3.31 ms)
+constexpr int COLOUR_ITEMS = 4;
+
 // Sub-chunks of events and groups of helicity rows sized to the caller's workspace:
 // the largest helicity group that still leaves a sub-chunk of min(nev, 65536) events
 // (enough waves for every SIMD), then as many events as the workspace holds.
@@ -910,8 +916,6 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
   for (int64_t off = 0; off < s.nev; off += nsub) {
     const int64_t n = s.nev - off < nsub ? s.nev - off : nsub;
     const int64_t tiles = (n + 15) / 16, blocks = (n + 63) / 64;
-    int64_t cblk = (tiles + 3) / 4;
-    if (cblk > 65536) cblk = 65536;
     for (int h0 = 0; h0 < nrows; h0 += hg) {
       OrderedArgs a;
       a.s = s;
@@ -933,12 +937,18 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
       if (precision == 64 && a.cper > T::NG) a.cper = (a.cper + T::NG - 1) / T::NG * T::NG;
       a.cparts = (count + a.cper - 1) / a.cper;
       a.cper *= unit;
-      // ranges of helicity rows of the colour sum: as many as give every SIMD two waves
+      // The colour sum's waves take (tile, range of rows) items in turn, so that a block stages its
+      // matrix once: as many blocks as a CU holds (61 KB of matrix each at 120 colours: two).
+      // The rows are split until every wave has COLOUR_ITEMS items, so that few events fill the
+      // chip and the last round of many is short.
+      const int64_t cslots = (int64_t)cus * (T::NCOLOR > 64 ? 2 : 8);
       int hper = hg;
-      while (hper > 1 && tiles * (hg / hper) < 8ll * cus) hper /= 2;
+      while (hper > 1 && tiles * (hg / hper) < COLOUR_ITEMS * 4 * cslots) hper /= 2;
       const int hparts = (hg + hper - 1) / hper;
+      int64_t cblk = (tiles * hparts + 3) / 4;
+      if (cblk > cslots) cblk = cslots;
       const int acc = h0 > 0;
-      const dim3 gj((unsigned)blocks, (unsigned)(ng * a.cparts)), gc((unsigned)cblk, (unsigned)hparts);
+      const dim3 gj((unsigned)blocks, (unsigned)(ng * a.cparts)), gc((unsigned)cblk);
       const int64_t step = (int64_t)hper * T::NCOLOR * a.ld;
       const dim3 gs((unsigned)tiles);
       if (precision == 32) {
