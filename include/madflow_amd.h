@@ -283,6 +283,13 @@ int mfx_vegas_refine(double* grid, const double* hist, int ndim, int nbins, doub
  * iteration) with key (seed, 0x6d66).  keep (nev,) u8 device; index_out (nev,) i32 device
  * receives the kept event indices in order; *nkeep_host (optional, synchronises) their
  * number.  Events with w > wmax are kept with weight w / wmax, the others with weight 1. */
+/* x1, x2 and the dynamic scale of the npass passing events of a hadronic generation call, in
+ * their compact order: x_out f64 [2][npass]; q2_out f64 (npass,) or NULL, the square of half the
+ * sum of the outgoing transverse masses sqrt(E^2 - pz^2) (madflow_exec.py:427-430), from dense
+ * (npass, nexternal, 4).  slot (nev,) and x12 (nev, 2) as mfx_ps_generate / mfx_mc_generate
+ * wrote them. */
+int mfx_hadronic_points(const double* dense, const int* slot, const double* x12, int64_t nev, int64_t npass,
+                        int nexternal, double* x_out, double* q2_out, void* stream);
 int64_t mfx_unweight_workspace_size(int64_t nev);
 int mfx_unweight(const double* w, int64_t nev, double wmax, uint32_t seed, uint32_t iteration, uint64_t ev0,
                  uint8_t* keep, int* index_out, void* workspace, int64_t workspace_bytes, int64_t* nkeep_host,

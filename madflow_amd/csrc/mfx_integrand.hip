@@ -734,6 +734,37 @@ __global__ void __launch_bounds__(GEN_BLOCK) k_compact(int nexternal, int64_t ne
   }
 }
 
+// a^2 - b^2 with both squares rounded, as elementwise operations round them: contracted into
+// one, the difference of a soft leg far along z would differ by its cancellation
+__device__ __forceinline__ double square_difference(double a, double b) {
+#pragma clang fp contract(off)
+  const double a2 = a * a, b2 = b * b;
+  return a2 - b2;
+}
+
+// x1, x2 (two planes of npass) and the dynamic scale Q^2 = (sum of the outgoing transverse
+// masses / 2)^2 of the passing events, in their compact order.  Bound by the launch at the
+// 1e5 points of an iteration; selecting by mask and forming Q^2 elementwise took 20 launches and
+// two waits of the host for the mask's count.
+__global__ void __launch_bounds__(GEN_BLOCK) k_hadronic_points(const double* __restrict__ dense,
+                                                               const int* __restrict__ slot,
+                                                               const double* __restrict__ x12, int64_t nev,
+                                                               int64_t npass, int nexternal,
+                                                               double* __restrict__ x_out,
+                                                               double* __restrict__ q2_out) {
+  const int64_t e = (int64_t)blockIdx.x * GEN_BLOCK + threadIdx.x;
+  if (e >= nev) return;
+  const int s = slot[e];
+  if (s < 0 || s >= npass) return;
+  x_out[s] = x12[2 * e];
+  x_out[npass + s] = x12[2 * e + 1];
+  if (!q2_out) return;
+  const double* d = dense + (int64_t)s * nexternal * 4;
+  double mt = 0.0;
+  for (int l = 2; l < nexternal; ++l) mt += sqrt(fmax(square_difference(d[4 * l], d[4 * l + 3]), 0.0));
+  q2_out[s] = 0.25 * mt * mt;
+}
+
 // ---------------------------------------------------------------- accumulation
 // partial layout per block: NSCAL scalars then ndim*nbins histogram (plain sums) and the
 // same number of compensation terms.
@@ -1297,6 +1328,17 @@ int mfx_vegas_refine(double* grid, const double* hist, int ndim, int nbins, doub
   if (ndim < 1 || ndim > MAXDIM || nbins < 2 || nbins > MAXBINS) return fail(-2, "ndim/nbins out of range%s", "");
   if (!grid || !hist) return fail(-3, "null pointer%s", "");
   hipLaunchKernelGGL(k_refine, dim3(ndim), dim3(64), 0, (hipStream_t)stream, grid, hist, nbins, alpha);
+  return hip_status(hipGetLastError());
+}
+
+int mfx_hadronic_points(const double* dense, const int* slot, const double* x12, int64_t nev, int64_t npass,
+                        int nexternal, double* x_out, double* q2_out, void* stream) {
+  if (nev < 0 || nev > 0x7fffffff || npass < 0 || npass > nev) return fail(-2, "need 0 <= npass <= nev < 2^31%s", "");
+  if (nexternal < 4 || nexternal > RAMBO_MAXN + 2) return fail(-2, "nexternal must lie in [4, 10]%s", "");
+  if (npass == 0) return 0;
+  if (!dense || !slot || !x12 || !x_out) return fail(-3, "null pointer%s", "");
+  hipLaunchKernelGGL(k_hadronic_points, dim3((unsigned)((nev + GEN_BLOCK - 1) / GEN_BLOCK)), dim3(GEN_BLOCK), 0,
+                     (hipStream_t)stream, dense, slot, x12, nev, npass, nexternal, x_out, q2_out);
   return hip_status(hipGetLastError());
 }
 

@@ -55,11 +55,14 @@ def process_index(name):
     return idx
 
 
+_Two, _Six = ctypes.c_double * 2, ctypes.c_double * 6
+
+
 def _as_scalar(x, name):
     if isinstance(x, torch.Tensor):
         if x.numel() != 1:
             raise ValueError("%s must be a scalar" % name)
-        return x.reshape(()).item()
+        return x.item()
     return x
 
 
@@ -80,6 +83,7 @@ class MatrixBase:
         self.kernel_family = kernels or self.kernels[0]
         self._idx = None
         self._ws = {}
+        self._no_ws = False
 
     @property
     def registry_name(self):
@@ -104,9 +108,10 @@ class MatrixBase:
             raise TypeError("%s.smatrix expects %d model parameters %s" % (
                 type(self).__name__, len(self.params), list(self.params)))
         vals = dict(zip(self.params, params))
-        mw = np.array([float(_as_scalar(vals["mdl_MT"], "mdl_MT")), float(_as_scalar(vals["mdl_WT"], "mdl_WT"))])
-        gc = np.zeros(6)
-        per_event = None
+        # host arrays of the C call: (mass, width) and (re, im) of GC_10, GC_11, GC_12
+        mw = _Two(float(_as_scalar(vals["mdl_MT"], "mdl_MT")), float(_as_scalar(vals["mdl_WT"], "mdl_WT")))
+        gc = _Six()
+        running = {}
         for name, slot in _GC_SLOT.items():
             if name not in vals:
                 continue
@@ -114,21 +119,20 @@ class MatrixBase:
             if isinstance(v, torch.Tensor) and v.numel() > 1:
                 if v.numel() != nev:
                     raise ValueError("%s must have length 1 or nev=%d" % (name, nev))
-                if per_event is None:
-                    per_event = torch.zeros((3, nev, 2), dtype=torch.float64, device=all_ps.device)
-                vv = v.to(device=all_ps.device, dtype=torch.complex128).reshape(-1)
-                per_event[slot, :, 0] = vv.real
-                per_event[slot, :, 1] = vv.imag
+                running[slot] = v.to(device=all_ps.device, dtype=torch.complex128).reshape(-1)
             else:
                 c = complex(_as_scalar(v, name))
                 gc[2 * slot] = c.real
                 gc[2 * slot + 1] = c.imag
-        if per_event is not None:
-            # broadcast frozen couplings into the per-event array too
-            for name, slot in _GC_SLOT.items():
-                if name in vals and not (isinstance(vals[name], torch.Tensor) and vals[name].numel() > 1):
-                    per_event[slot, :, 0] = gc[2 * slot]
-                    per_event[slot, :, 1] = gc[2 * slot + 1]
+        per_event = None
+        if running:
+            # the planes [3][nev] (re, im) in one copy, frozen couplings broadcast into theirs
+            planes = [running.get(slot) for slot in range(3)]
+            for slot, plane in enumerate(planes):
+                if plane is None:
+                    planes[slot] = torch.full((), complex(gc[2 * slot], gc[2 * slot + 1]), dtype=torch.complex128,
+                                              device=all_ps.device).expand(nev)
+            per_event = torch.stack(planes)
         return all_ps, nev, mw, gc, per_event
 
     # device workspace for processes evaluated by the colour-ordered kernels: at most this
@@ -140,10 +144,13 @@ class MatrixBase:
         process needs none.  One workspace is kept per (device, current stream) and is
         allocated while that stream is current, so the caching allocator orders its reuse
         after that stream's work, and calls on different streams never share one."""
+        if self._no_ws:
+            return None, 0
         lib = _lib.load()
         need = int(lib.mfx_smatrix_workspace_size(self.index, nev, self.precision, int(per_helicity)))
         if need < 0:
             _lib.check(need)
+        self._no_ws = need == 0 and nev > 0      # the process stages nothing, whatever the call
         if need == 0:
             return None, 0
         size = min(need, self.workspace_limit)
@@ -152,7 +159,7 @@ class MatrixBase:
         if ws is None or ws.numel() < size:
             self._ws.pop(key, None)
             ws = self._ws[key] = torch.empty(size, dtype=torch.uint8, device=device)
-        return ctypes.c_void_p(ws.data_ptr()), ws.numel()
+        return ws.data_ptr(), ws.numel()
 
     def _smatrix(self, all_ps, params):
         all_ps, nev, mw, gc, per_event = self._prepare(all_ps, params)
@@ -162,11 +169,9 @@ class MatrixBase:
         lib = _lib.load()
         ws, ws_bytes = self._workspace(nev, False, all_ps.device)
         _lib.check(lib.mfx_smatrix(
-            self.index, ctypes.c_void_p(all_ps.data_ptr()), nev, mw.ctypes.data_as(ctypes.c_void_p),
-            gc.ctypes.data_as(ctypes.c_void_p),
-            ctypes.c_void_p(per_event.data_ptr()) if per_event is not None else None,
-            ctypes.c_void_p(out.data_ptr()), self.precision, int(self.ref_compat), ws, ws_bytes,
-            _lib.stream_ptr(all_ps.device)))
+            self.index, all_ps.data_ptr(), nev, mw, gc, per_event.data_ptr() if per_event is not None else None,
+            out.data_ptr(), self.precision, int(self.ref_compat), ws, ws_bytes,
+            torch.cuda.current_stream(all_ps.device).cuda_stream))
         return out
 
     def _matrix(self, all_ps, hel, params, return_jamp=False):
@@ -182,11 +187,10 @@ class MatrixBase:
             lib = _lib.load()
             ws, ws_bytes = self._workspace(nev, True, all_ps.device)
             _lib.check(lib.mfx_matrix(
-                self.index, ctypes.c_void_p(all_ps.data_ptr()), nev, helv.ctypes.data_as(ctypes.c_void_p),
-                mw.ctypes.data_as(ctypes.c_void_p), gc.ctypes.data_as(ctypes.c_void_p),
-                ctypes.c_void_p(per_event.data_ptr()) if per_event is not None else None,
-                ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(jamp.data_ptr()) if jamp is not None else None,
-                self.precision, int(self.ref_compat), ws, ws_bytes, _lib.stream_ptr(all_ps.device)))
+                self.index, all_ps.data_ptr(), nev, helv.ctypes.data_as(ctypes.c_void_p), mw, gc,
+                per_event.data_ptr() if per_event is not None else None, out.data_ptr(),
+                jamp.data_ptr() if jamp is not None else None, self.precision, int(self.ref_compat), ws, ws_bytes,
+                _lib.stream_ptr(all_ps.device)))
         if return_jamp:
             return out, torch.complex(jamp[..., 0], jamp[..., 1])
         return out

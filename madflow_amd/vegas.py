@@ -278,7 +278,7 @@ class MEIntegrand:
         self.last_chunk_npass = npass
         if len(self.subprocesses) > 1:
             return self._chunk_sum(b, ev0, n, iteration, keep_f, y_in, npass, s)
-        params, f_in = self.params, None
+        params = self.params
         if self.hadronic and npass:
             params, lumi = self._hadronic_factors(b, n, npass)
         if self.me_timer is not None and npass:
@@ -292,15 +292,13 @@ class MEIntegrand:
             # with no passing event every slot is -1 and nothing reads the matrix elements, but
             # the library still needs a device pointer, which an empty tensor does not have
             me = self.matrix.smatrix(b["dense"][:npass], *params) if npass else b["wps"][:1]
-        if self.hadronic:
-            # f = luminosity x |M|^2 x weight (madflow_exec.py:455-459), scattered to full length
-            f_in = torch.zeros(n, dtype=torch.float64, device=self.device)
-            if npass:
-                ok = b["flag"][:n] == 1
-                f_in[ok] = me * lumi * b["wps"][:n][ok]
+        if self.hadronic and npass:
+            # f = luminosity x |M|^2 x weight (madflow_exec.py:455-459); the accumulation
+            # multiplies the weights of the passing events
+            me = me * lumi
         _lib.check(self.lib.mfx_vegas_accumulate(
             ctypes.byref(self.p), ev0, n, iteration, _ptr(y_in), _ptr(b["slot"]), _ptr(me), _ptr(b["wps"]),
-            _ptr(f_in), _ptr(b["f"]) if keep_f else None, _ptr(b["ws"]), b["ws"].numel(), _ptr(b["result"]), s))
+            None, _ptr(b["f"]) if keep_f else None, _ptr(b["ws"]), b["ws"].numel(), _ptr(b["result"]), s))
         return b["result"].cpu().numpy().copy(), npass, (b["f"][:n] if keep_f else None)
 
     def unweight(self, w, wmax, iteration, ev0=0):
@@ -391,20 +389,21 @@ class MEIntegrand:
         running alpha_s is given, and x1 f(x1) x2 f(x2) / (x1 x2) at Q^2, for the process
         ``sub`` (an entry of subprocesses; the first by default)."""
         _, model, params0, flavours = sub if sub is not None else self.subprocesses[0]
-        d = b["dense"][:npass]
-        x = b["x12"][:n][b["flag"][:n] == 1]
-        if self.scale is None:
-            out = d[:, 2:, :]
-            mt = torch.sqrt(torch.clamp(out[..., 0] ** 2 - out[..., 3] ** 2, min=0.0)).sum(dim=1)
-            q2 = (0.5 * mt) ** 2
-        else:
-            q2 = torch.full((npass,), float(self.scale) ** 2, dtype=torch.float64, device=self.device)
+        # x1, x2 and the dynamic scale of the passing events in one kernel: a boolean mask would
+        # wait for the device to count them
+        x = torch.empty((2, npass), dtype=torch.float64, device=self.device)
+        q2 = torch.empty(npass, dtype=torch.float64, device=self.device)
+        _lib.check(self.lib.mfx_hadronic_points(
+            _ptr(b["dense"]), _ptr(b["slot"]), _ptr(b["x12"]), n, npass, self.nexternal, _ptr(x),
+            _ptr(q2) if self.scale is None else None, _lib.stream_ptr(self.device)))
+        if self.scale is not None:
+            q2.fill_(float(self.scale) ** 2)
         params = params0
         if self.alphas is not None:
             params = list(model.evaluate(self.alphas(q2).to(torch.float64).reshape(-1)))
             if self.width is not None:
                 params[1] = float(self.width)
-        x1, x2 = x[:, 0], x[:, 1]
+        x1, x2 = x[0], x[1]
         if flavours is None:
             lumi = self.pdf(x1, q2) * self.pdf(x2, q2) / (x1 * x2)
         else:

@@ -79,3 +79,38 @@ def test_compaction_offsets(dev, n):
     w = torch.from_numpy(_tensors(n, 0)[0]).to(dev)
     idx, keep = unweight(w, 4.0, seed=3)
     assert torch.equal(idx.long(), torch.nonzero(keep).reshape(-1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("process", ["gg_ttx", "gg_ttxgg"])
+@pytest.mark.parametrize("n", [1, 257, 70001])
+def test_hadronic_points(dev, process, n):
+    """x1, x2 and Q^2 of the passing events, in their order, against selection by mask."""
+    print("hadronic points", process, n, flush=True)
+    ig = MEIntegrand(process, 13000.0, mapping="hadronic", pdf=lambda x, q2: x, seed=9)
+    ig.register_cut("pt", particle=2, min_val=100.0)
+    _, npass, _ = ig.chunk(0, n, 1)
+    b = ig._bufs
+    ok = b["flag"][:n] == 1
+    x, q2 = torch.empty((2, npass), dtype=torch.float64, device=dev), torch.empty(npass, dtype=torch.float64, device=dev)
+    _lib.check(ig.lib.mfx_hadronic_points(_ptr(b["dense"]), _ptr(b["slot"]), _ptr(b["x12"]), n, npass, ig.nexternal,
+                                          _ptr(x), _ptr(q2), _lib.stream_ptr(dev)))
+    assert torch.equal(x.T, b["x12"][:n][ok])
+    out = b["all_ps"][:n][ok][:, 2:]
+    mt = torch.sqrt(torch.clamp(out[..., 0] ** 2 - out[..., 3] ** 2, min=0.0)).sum(1)
+    # E^2 - pz^2 loses (E / mT)^2 in the contraction of its products
+    tol = 4e-16 * (1.0 + (out[..., 0] ** 2).sum(1) / mt ** 2)
+    assert bool(((q2 / (0.5 * mt) ** 2 - 1).abs() <= 8 * tol).all())
+
+
+@pytest.mark.gpu
+def test_running_and_frozen_couplings_mixed(dev):
+    """A coupling of one value beside couplings per event is broadcast into its plane."""
+    from madflow_amd.matrix import load_matrix
+    from madflow_amd.phasespace_gpu import sample_momenta
+    m, _ = load_matrix("gg_ttxg", precision=64)
+    ps = sample_momenta("gg_ttxg", 257, device=dev)
+    one = lambda v: torch.full((257,), v, dtype=torch.complex128, device=dev)
+    whole = m.smatrix(ps, 173.0, 1.5, one(-1.2), one(1.2j), one(1.44j))
+    assert torch.equal(m.smatrix(ps, 173.0, 1.5, -1.2, one(1.2j), torch.tensor([1.44j], dtype=torch.complex128)), whole)
+    assert torch.equal(m.smatrix(ps, 173.0, 1.5, one(-1.2), torch.tensor([1.2j], dtype=torch.complex128, device=dev), one(1.44j).cpu()), whole)
