@@ -24,18 +24,25 @@ struct RamboConst {
   double inorm;   // 1 / (2 pi)^(3n-4)
 };
 
+// N: the number of outgoing particles where it is a compile-time constant (momenta then stay in
+// registers), 0 where it is rc.n.
+template <int N> __device__ __forceinline__ int legs_of(const RamboConst& rc) { return N ? N : rc.n; }
+
 // Newton iterations allowed for the massive rescaling factor xi
 constexpr int NEWTON_MAX = 50;
 
+template <int N>
 __device__ __forceinline__ double massive_rescale(const RamboConst& rc, double sqrts, double (*p)[4], bool& converged);
 
 // x: 4n uniforms (cos theta, phi, and two for the energy) per particle; returns weight.
 // converged: false when the massive rescaling's Newton iteration did not reach
 // |sum E - sqrts| <= 1e-14 sqrts in NEWTON_MAX steps (the event is then off shell).
+template <int N = 0>
 __device__ __forceinline__ double rambo_event(const RamboConst& rc, const double* x, double sqrts,
                                               double (*p)[4], bool& converged) {
-  const int n = rc.n;
+  const int n = legs_of<N>(rc);
   double Q[4] = {0, 0, 0, 0};
+#pragma clang loop unroll_count(N ? 8 : 1)
   for (int i = 0; i < n; ++i) {
     const double costh = 2.0 * x[4 * i] - 1.0;
     const double sinth = sqrt(1.0 - costh * costh);
@@ -46,6 +53,7 @@ __device__ __forceinline__ double rambo_event(const RamboConst& rc, const double
     p[i][1] = e * sinth * sphi;
     p[i][2] = e * sinth * cphi;
     p[i][3] = e * costh;
+#pragma clang loop unroll_count(N ? 8 : 1)
     for (int k = 0; k < 4; ++k) Q[k] += p[i][k];
   }
   const double M = sqrt(Q[0] * Q[0] - (Q[1] * Q[1] + Q[2] * Q[2] + Q[3] * Q[3]));
@@ -54,6 +62,7 @@ __device__ __forceinline__ double rambo_event(const RamboConst& rc, const double
   const double b1 = -Q[1] * iM, b2 = -Q[2] * iM, b3 = -Q[3] * iM;
   const double gamma = Q[0] * iM;
   const double a = 1.0 / (1.0 + gamma);
+#pragma clang loop unroll_count(N ? 8 : 1)
   for (int i = 0; i < n; ++i) {
     const double bq = p[i][1] * b1 + p[i][2] * b2 + p[i][3] * b3;
     const double t = bq * a + p[i][0];
@@ -64,7 +73,7 @@ __device__ __forceinline__ double rambo_event(const RamboConst& rc, const double
   }
   double logw = rc.logw0 + (2 * n - 4) * log(sqrts);
   converged = true;
-  if (rc.massive) logw += massive_rescale(rc, sqrts, p, converged);
+  if (rc.massive) logw += massive_rescale<N>(rc, sqrts, p, converged);
   return exp(logw) * rc.inorm;
 }
 
@@ -72,8 +81,9 @@ __device__ __forceinline__ double rambo_event(const RamboConst& rc, const double
 // xi with sum_i sqrt(m_i^2 + xi^2 E_i^2) = sqrts; returns the log of the weight factor
 // xi^(2n-3) prod(|p_i|/E_i) / sum(|p_i|^2/E_i) * sqrts.  Needs sum m_i < sqrts (the
 // callers check it); converged reports whether Newton met its tolerance.
+template <int N>
 __device__ __forceinline__ double massive_rescale(const RamboConst& rc, double sqrts, double (*p)[4], bool& converged) {
-  const int n = rc.n;
+  const int n = legs_of<N>(rc);
   double logw = 0.0;
   converged = false;
   {
@@ -82,6 +92,7 @@ __device__ __forceinline__ double massive_rescale(const RamboConst& rc, double s
     for (int it = 0; it < NEWTON_MAX; ++it) {
       const double x2 = xi * xi;
       double f0 = -sqrts, g0 = 0.0;
+#pragma clang loop unroll_count(N ? 8 : 1)
       for (int i = 0; i < n; ++i) {
         const double E2 = p[i][0] * p[i][0];
         const double nE = sqrt(rc.masses[i] * rc.masses[i] + E2 * x2);
@@ -96,6 +107,7 @@ __device__ __forceinline__ double massive_rescale(const RamboConst& rc, double s
     }
     const double x2 = xi * xi;
     double wt2 = 1.0, wt3 = 0.0;
+#pragma clang loop unroll_count(N ? 8 : 1)
     for (int i = 0; i < n; ++i) {
       const double v = p[i][0] * xi;
       const double nE = sqrt(rc.masses[i] * rc.masses[i] + p[i][0] * p[i][0] * x2);
@@ -134,11 +146,13 @@ __device__ __host__ inline double diet_solve(double r, int k) {
 // whose invariant masses are drawn from their exact marginal densities; massive
 // particles are then obtained with RAMBO's xi rescaling.  x[0..n-3] fix the masses,
 // x[n-2+2i], x[n-1+2i] the decay angles of step i.
+template <int N = 0>
 __device__ __forceinline__ double diet_event(const RamboConst& rc, const double* x, double sqrts, double (*p)[4],
                                              bool& converged) {
-  const int n = rc.n;
+  const int n = legs_of<N>(rc);
   double Q[4] = {sqrts, 0.0, 0.0, 0.0};
   double M = sqrts;
+#pragma clang loop unroll_count(N ? 8 : 1)
   for (int i = 0; i < n - 1; ++i) {
     double Mn = 0.0;
     if (i < n - 2) Mn = M * sqrt(diet_solve(x[i], n - 2 - i));
@@ -156,13 +170,15 @@ __device__ __forceinline__ double diet_event(const RamboConst& rc, const double*
     p[i][1] = k1 + b1 * c;
     p[i][2] = k2 + b2 * c;
     p[i][3] = k3 + b3 * c;
+#pragma clang loop unroll_count(N ? 8 : 1)
     for (int j = 0; j < 4; ++j) Q[j] -= p[i][j];
     M = Mn;
   }
+#pragma clang loop unroll_count(N ? 8 : 1)
   for (int j = 0; j < 4; ++j) p[n - 1][j] = Q[j];
   double logw = rc.logw0 + (2 * n - 4) * log(sqrts);
   converged = true;
-  if (rc.massive) logw += massive_rescale(rc, sqrts, p, converged);
+  if (rc.massive) logw += massive_rescale<N>(rc, sqrts, p, converged);
   return exp(logw) * rc.inorm;
 }
 

@@ -114,3 +114,29 @@ def test_running_and_frozen_couplings_mixed(dev):
     whole = m.smatrix(ps, 173.0, 1.5, one(-1.2), one(1.2j), one(1.44j))
     assert torch.equal(m.smatrix(ps, 173.0, 1.5, -1.2, one(1.2j), torch.tensor([1.44j], dtype=torch.complex128)), whole)
     assert torch.equal(m.smatrix(ps, 173.0, 1.5, one(-1.2), torch.tensor([1.2j], dtype=torch.complex128, device=dev), one(1.44j).cpu()), whole)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_out", [2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("massive", [False, True])
+def test_generation_by_number_of_legs(dev, n_out, massive):
+    """The generation kernels of two to five legs and the general one against RAMBO at each
+    event's partonic energy, with a cut on the last leg."""
+    from madflow_amd.phasespace_gpu import PhaseSpaceGenerator, rambo
+    print("legs", n_out, massive, flush=True)
+    masses = [173.0 if massive and i < 2 else 0.0 for i in range(n_out)]
+    gen = PhaseSpaceGenerator(n_out + 2, 13000.0, masses=masses)
+    gen.p.shat_min = 2000.0 ** 2
+    x = torch.rand((1025, gen.ndim), generator=torch.Generator().manual_seed(n_out), dtype=torch.float64).to(dev)
+    ps, w, x1, x2, _ = gen.generate(x)
+    p, wr = rambo(x[:, 2:].contiguous(), n_out, torch.sqrt(x1 * x2) * 13000.0, masses=masses)
+    scale = (x1 * x2).sqrt() * 13000.0
+    # sqrt(x1 x2) s is rounded once more here; a Newton step ends at 1e-14 of the energy
+    assert ((ps[:, 2:] - p).abs().amax((1, 2)) / scale).max().item() < 1e-12
+    tau = x1 * x2
+    jac = (1.0 - (2000.0 / 13000.0) ** 2) * -torch.log(tau) * 389379365.6 / (2.0 * tau * 13000.0 ** 2)
+    assert ((w / (wr * jac)) - 1).abs().max().item() < 1e-11
+    gen.register_cut("pt", particle=n_out + 1, min_val=300.0)
+    cut, _, _, _, idx = gen(x)
+    want = torch.nonzero(torch.hypot(ps[:, -1, 1], ps[:, -1, 2]) > 300.0)
+    assert torch.equal(idx.long(), want) and torch.equal(cut, ps[want[:, 0]])
