@@ -11,7 +11,7 @@ import torch
 
 from madflow_amd import _lib
 from madflow_amd.multichannel import MultiChannelIntegrand
-from madflow_amd.phasespace_gpu import philox_uniforms
+from madflow_amd.phasespace_gpu import PhaseSpaceGenerator, philox_uniforms, rambo
 from madflow_amd.vegas import MEIntegrand, _ptr
 from oracle import oracle as O
 
@@ -40,6 +40,39 @@ def test_accumulate_sums_and_histogram(dev, n, nbins):
     tol = (n / (4.0 * min(1024, -(-n // 256))) + 64) * 2.0 ** -53 + 1e-13
     for d in range(ig.ndim):
         hist = np.bincount((y[:, d] * nbins).astype(int), weights=f * f, minlength=nbins)
+        np.testing.assert_allclose(r[6 + d * nbins:6 + (d + 1) * nbins], hist, rtol=tol)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 65, 300001])
+@pytest.mark.parametrize("n_out,mapping,ndim,nbins", [(3, 1, 5, 64), (4, 0, 16, 3), (5, 2, 22, 50), (7, 2, 30, 16)])
+def test_accumulate_of_an_external_proposal(dev, n_out, mapping, ndim, nbins, n):
+    """Odd and large numbers of dimensions, one copy of the histogram a wave (22 of 50 bins) and
+    two; coordinates at and beyond the ends of the range and not finite, weights not finite."""
+    print("external", ndim, nbins, n, flush=True)
+    gen = PhaseSpaceGenerator(n_out + 2, 13000.0)
+    p = gen.p
+    p.mapping, p.ndim, p.nbins = mapping, ndim, nbins
+    rng = np.random.default_rng(n + ndim)
+    y = rng.random((n, ndim), dtype=np.float32)
+    f = rng.exponential(size=n)
+    y[::7, 0], y[::5, 1], y[::11, 2], y[::13, 3], y[::17, 4] = 1.0, -0.5, 1.5, np.nan, np.inf
+    f[3::9], f[5::31] = np.nan, np.inf
+    yd, fd, fo = torch.from_numpy(y).to(dev), torch.from_numpy(f).to(dev), torch.empty(n, dtype=torch.float64, device=dev)
+    ws = torch.empty(gen.lib.mfx_integrand_workspace_size(n, ndim, nbins), dtype=torch.uint8, device=dev)
+    out = torch.empty(6 + ndim * nbins, dtype=torch.float64, device=dev)
+    _lib.check(gen.lib.mfx_vegas_accumulate(ctypes.byref(p), 0, n, 0, _ptr(yd), None, None, None, _ptr(fd), _ptr(fo),
+                                            _ptr(ws), ws.numel(), _ptr(out), _lib.stream_ptr(dev)))
+    r = out.cpu().numpy()
+    f = np.where(np.isfinite(f), f, 0.0)
+    assert np.array_equal(fo.cpu().numpy(), f)
+    np.testing.assert_allclose(r[:2], [math.fsum(f), math.fsum(f * f)], rtol=4e-16 * np.log2(n + 2) + 1e-15)
+    assert r[2] == f.max() and r[3] == np.count_nonzero(f)
+    yc = np.clip(np.where(np.isfinite(y), y, 0.0).astype(np.float64), 0.0, 1.0)
+    tol = (n / (4.0 * min(1024, -(-n // 256))) + 64) * 2.0 ** -53 + 1e-13
+    for d in range(ndim):
+        bins = np.minimum((yc[:, d] * nbins).astype(int), nbins - 1)
+        hist = np.bincount(bins, weights=f * f, minlength=nbins)
         np.testing.assert_allclose(r[6 + d * nbins:6 + (d + 1) * nbins], hist, rtol=tol)
 
 
@@ -122,7 +155,6 @@ def test_running_and_frozen_couplings_mixed(dev):
 def test_generation_by_number_of_legs(dev, n_out, massive):
     """The generation kernels of two to five legs and the general one against RAMBO at each
     event's partonic energy, with a cut on the last leg."""
-    from madflow_amd.phasespace_gpu import PhaseSpaceGenerator, rambo
     print("legs", n_out, massive, flush=True)
     masses = [173.0 if massive and i < 2 else 0.0 for i in range(n_out)]
     gen = PhaseSpaceGenerator(n_out + 2, 13000.0, masses=masses)
