@@ -123,15 +123,13 @@ struct SplineEval {
   float z, ld;  // output and log derivative
 };
 
-__device__ __forceinline__ SplineEval rq_forward(const float* raw, float x) {
-  float w[K], h[K];
-  softmax_bins(raw, MINW, w);
-  softmax_bins(raw + K, MINH, h);
+// w, h: the bins; rd: the K + 1 raw derivatives
+__device__ __forceinline__ SplineEval rq_forward(const float* w, const float* h, const float* rd, float x) {
   x = fminf(fmaxf(x, 0.f), 1.f);
   const Edge ex = bin_of(w, x);
   const int k = ex.k;
   const Edge ey = edges_at(h, k);
-  const float a = MIND + softplus(raw[2 * K + k]), c = MIND + softplus(raw[2 * K + k + 1]);
+  const float a = MIND + softplus(rd[k]), c = MIND + softplus(rd[k + 1]);
   const float wk = ex.hi - ex.lo, hk = ey.hi - ey.lo;
   const float xi = fminf(fmaxf((x - ex.lo) / wk, 0.f), 1.f);
   const float s = hk / wk;
@@ -145,15 +143,12 @@ __device__ __forceinline__ SplineEval rq_forward(const float* raw, float x) {
   return r;
 }
 
-__device__ __forceinline__ SplineEval rq_inverse(const float* raw, float z) {
-  float w[K], h[K];
-  softmax_bins(raw, MINW, w);
-  softmax_bins(raw + K, MINH, h);
+__device__ __forceinline__ SplineEval rq_inverse(const float* w, const float* h, const float* rd, float z) {
   z = fminf(fmaxf(z, 0.f), 1.f);
   const Edge ey = bin_of(h, z);
   const int k = ey.k;
   const Edge ex = edges_at(w, k);
-  const float a = MIND + softplus(raw[2 * K + k]), c = MIND + softplus(raw[2 * K + k + 1]);
+  const float a = MIND + softplus(rd[k]), c = MIND + softplus(rd[k + 1]);
   const float wk = ex.hi - ex.lo, hk = ey.hi - ey.lo;
   const float s = hk / wk;
   const float d = z - ey.lo;
@@ -171,6 +166,20 @@ __device__ __forceinline__ SplineEval rq_inverse(const float* raw, float z) {
   r.z = ex.lo + xi * wk;                                          // x
   r.ld = -(2.f * __logf(s) + __logf(P) - 2.f * __logf(den));     // log|dx/du|
   return r;
+}
+
+__device__ __forceinline__ SplineEval rq_forward(const float* raw, float x) {
+  float w[K], h[K];
+  softmax_bins(raw, MINW, w);
+  softmax_bins(raw + K, MINH, h);
+  return rq_forward(w, h, raw + 2 * K, x);
+}
+
+__device__ __forceinline__ SplineEval rq_inverse(const float* raw, float z) {
+  float w[K], h[K];
+  softmax_bins(raw, MINW, w);
+  softmax_bins(raw + K, MINH, h);
+  return rq_inverse(w, h, raw + 2 * K, z);
 }
 
 // Gradient of gz*z + gl*ld w.r.t. the raw parameters (written to graw[NPD]) and x.
@@ -531,17 +540,25 @@ k_flow(FlowArgs A, const float* __restrict__ P,
 // the spline runs on full waves, a sample per lane and a transformed dimension per wave,
 // instead of on one wave of eight.  For that, wave w computes the spline parameters of
 // dimension w, w + 4, ... of all 64 samples itself (four 16-column tiles from the
-// dimension's first column), so that they only pass through its own part of LDS.  Each
-// output element sums the same products in the same order as in k_flow: the results are
-// equal to the last bit.  76 KB of LDS: two blocks on a CU.
-// 1e6 samples of an 8-layer flow, inverse: 8 dimensions 7.14 -> 2.52 ms, 11 dimensions 14.6 -> 3.43 ms,
-// 4 dimensions (6 layers) 4.45 -> 1.63 ms.
+// dimension's first column), so that they only pass through its own part of LDS: a
+// 16-column tile at a time, the widths, the heights, then the derivatives, each read into
+// registers before the next is staged.  Each output element sums the same products in the same
+// order as in k_flow: the results are equal to the last bit.  What bounds it is latency: a
+// wave's layer is a chain of products, LDS and special functions between four barriers, and
+// neither the VALU nor the matrix cores are busy half of the time.  So it takes as many waves
+// as fit: 51 KB of LDS and 168 registers, three blocks on a CU (two with all 49 parameters
+// of a sample staged at once, 79 KB; the products of W3 are unrolled twice only, as more spills).
+// 1e6 samples of an 8-layer flow, inverse: 8 dimensions 7.14 ms in k_flow, 2.52 with two blocks on a CU,
+// 1.97 now; 11 dimensions 14.6, 3.43, 2.68 ms; 4 dimensions (6 layers) 4.45, 1.63, 1.29 ms.
 constexpr int WT = 64;          // samples per block
 constexpr int WV = 4;           // waves per block
 constexpr int XP = DMAX + 1;    // row pitch of the coordinates in LDS (a sample per lane)
+constexpr int RP = 21;          // row pitch of the staged spline parameters: a sample per lane reads
+                                // without conflicts, four rows apart start 20 banks apart
+static_assert(K == 16 && RP > K, "widths, heights and derivatives are staged a 16-column tile at a time");
 
 template <bool INV>
-__global__ void __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * WV) __attribute__((amdgpu_waves_per_eu(3)))
 k_flow_wide(FlowArgs A, const float* __restrict__ P, const unsigned short* __restrict__ Pb) {
   const int D = A.geo.D, L = A.geo.L;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -549,8 +566,8 @@ k_flow_wide(FlowArgs A, const float* __restrict__ P, const unsigned short* __res
   __shared__ float xs[WT * XP], ld_b[WT * XP];
   __shared__ __attribute__((aligned(16))) float xa[WT * DMAX];
   __shared__ __attribute__((aligned(16))) unsigned short h2s[WT * WP];
-  // the first hidden layer, then each wave's spline parameters
-  __shared__ __attribute__((aligned(16))) float raws[WV * WT * NPD];
+  // the first hidden layer, then a part of each wave's spline parameters
+  __shared__ __attribute__((aligned(16))) float raws[WV * WT * RP];
   unsigned short* h1s = reinterpret_cast<unsigned short*>(raws);
   static_assert(sizeof(raws) >= sizeof(h2s), "the hidden layer fits the parameters' space");
   const int64_t s0 = (int64_t)blockIdx.x * WT;
@@ -591,16 +608,16 @@ k_flow_wide(FlowArgs A, const float* __restrict__ P, const unsigned short* __res
 #pragma unroll
       for (int u = 0; u < NS; ++u) v[u] = b1;
       for (int i0 = 0; i0 < nA; i0 += 4) {
-        float w[4];
+        float w1[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = i0 + i < nA ? P[g.oW1 + (i0 + i) * H + j1] : 0.f;
+        for (int i = 0; i < 4; ++i) w1[i] = i0 + i < nA ? P[g.oW1 + (i0 + i) * H + j1] : 0.f;
 #pragma unroll
         for (int u = 0; u < NS; ++u) {
           const float4 x = *reinterpret_cast<const float4*>(xa + (sb + u) * DMAX + i0);
-          v[u] += x.x * w[0];
-          v[u] += x.y * w[1];
-          v[u] += x.z * w[2];
-          v[u] += x.w * w[3];
+          v[u] += x.x * w1[0];
+          v[u] += x.y * w1[1];
+          v[u] += x.z * w1[2];
+          v[u] += x.w * w1[3];
         }
       }
 #pragma unroll
@@ -630,47 +647,56 @@ k_flow_wide(FlowArgs A, const float* __restrict__ P, const unsigned short* __res
     }
     __syncthreads();
     // layer 3 and the spline, a transformed dimension per wave
-    float* raw = raws + wid * WT * NPD;
+    float* raw = raws + wid * WT * RP;
     for (int b = wid; b < nB; b += WV) {
       const int c0 = b * NPD;
-      f32x4 acc[WT / 16][4];
+      float bins[2][K];
 #pragma unroll
-      for (int m = 0; m < WT / 16; ++m)
+      for (int half = 0; half < 2; ++half) {     // widths and heights, then the derivatives
+        f32x4 acc[WT / 16][2];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc[m][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-      float b3[4];
-      const unsigned short* w3[4];
+        for (int m = 0; m < WT / 16; ++m) acc[m][0] = acc[m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        float b3[2];
+        const unsigned short* w3[2];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int col = c0 + 16 * u + r < NP ? c0 + 16 * u + r : NP - 1;   // columns past NPD are dropped
-        b3[u] = P[g.ob3 + col];
-        w3[u] = Pb + g.oW3t + col * H + k8;
-      }
+        for (int u = 0; u < 2; ++u) {
+          const int cu = c0 + 32 * half + 16 * u + r;
+          const int col = cu < NP ? cu : NP - 1;   // columns past NPD are dropped
+          b3[u] = P[g.ob3 + col];
+          w3[u] = Pb + g.oW3t + col * H + k8;
+        }
+#pragma unroll 2
+        for (int K0 = 0; K0 < H; K0 += 32) {
+          bf16x8 w[2];
 #pragma unroll
-      for (int K0 = 0; K0 < H; K0 += 32) {
-        bf16x8 w[4];
+          for (int u = 0; u < 2; ++u) w[u] = ld_bf16x8(w3[u] + K0);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) w[u] = ld_bf16x8(w3[u] + K0);
+          for (int m = 0; m < WT / 16; ++m) {
+            const bf16x8 a = ld_bf16x8(h2s + (16 * m + r) * WP + K0 + k8);
 #pragma unroll
-        for (int m = 0; m < WT / 16; ++m) {
-          const bf16x8 a = ld_bf16x8(h2s + (16 * m + r) * WP + K0 + k8);
+            for (int u = 0; u < 2; ++u) acc[m][u] = mfma_k32(a, w[u], acc[m][u]);
+          }
+        }
 #pragma unroll
-          for (int u = 0; u < 4; ++u) acc[m][u] = mfma_k32(a, w[u], acc[m][u]);
+        for (int u = 0; u < 2; ++u) {
+          if (u == 0 || half == 0) wave_sync();  // what was staged before is read
+          if (16 * u + 32 * half + r < NPD) {
+#pragma unroll
+            for (int m = 0; m < WT / 16; ++m)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) raw[(16 * m + kq + i) * RP + 16 * half * u + r] = acc[m][u][i] + b3[u];
+          }
+          if (half == 0) {
+            wave_sync();
+            softmax_bins(raw + lane * RP, u ? MINH : MINW, bins[u]);
+          }
         }
       }
-      wave_sync();                         // this wave's previous dimension is read
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (16 * u + r < NPD) {
-#pragma unroll
-          for (int m = 0; m < WT / 16; ++m)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) raw[(16 * m + kq + i) * NPD + 16 * u + r] = acc[m][u][i] + b3[u];
-        }
       wave_sync();
       const int d = g.B[b];
       const float x = xs[lane * XP + d];
-      const SplineEval sp = INV ? rq_inverse(raw + lane * NPD, x) : rq_forward(raw + lane * NPD, x);
+      const SplineEval sp = INV ? rq_inverse(bins[0], bins[1], raw + lane * RP, x)
+                                : rq_forward(bins[0], bins[1], raw + lane * RP, x);
       xs[lane * XP + d] = sp.z;
       ld_b[lane * XP + b] = sp.ld;
     }
@@ -1486,8 +1512,8 @@ static int nb_bound(const FlowGeom& G) {
 
 // Samples that k_flow's blocks hold at once (two tiles on a CU at up to 4 transformed
 // dimensions, else one): up to there its eight waves a tile end sooner, beyond it needs a second
-// round and k_flow_wide takes over.  8-dim flow, 8,192 samples: k_flow 65 us, k_flow_wide 72 us;
-// 16,384 samples: 125 us, 75 us.  11-dim flow, 4,000 samples: 69 us, 97 us; 8,192: 128 us, 97 us.
+// round and k_flow_wide takes over.  8-dim flow, 8,192 samples: k_flow 65 us, k_flow_wide 71 us;
+// 16,384 samples: 125 us, 73 us.  11-dim flow, 4,000 samples: 68 us, 98 us; 8,192: 128 us, 99 us.
 static int64_t flow_round(const FlowGeom& G) {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
