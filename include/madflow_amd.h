@@ -276,13 +276,6 @@ int mfx_mc_moments(int64_t nev, int nch, const int* slot, const double* me, cons
  * and equal-weight rebinning, per dimension (device grid updated in place). */
 int mfx_vegas_refine(double* grid, const double* hist, int ndim, int nbins, double alpha, void* stream);
 
-/* ------------------------------------------------ learned proposal (flow) */
-/* Hit-or-miss unweighting of nev weighted events (replaces handing them to MadGraph's
- * lhe_parser unweight, lhe_writer.py:319-356): keep event e with probability
- * min(1, w[e] / wmax), the uniform taken from the Philox stream (ev0 + e, 0xffffffff,
- * iteration) with key (seed, 0x6d66).  keep (nev,) u8 device; index_out (nev,) i32 device
- * receives the kept event indices in order; *nkeep_host (optional, synchronises) their
- * number.  Events with w > wmax are kept with weight w / wmax, the others with weight 1. */
 /* x1, x2 and the dynamic scale of the npass passing events of a hadronic generation call, in
  * their compact order: x_out f64 [2][npass]; q2_out f64 (npass,) or NULL, the square of half the
  * sum of the outgoing transverse masses sqrt(E^2 - pz^2) (madflow_exec.py:427-430), from dense
@@ -290,6 +283,14 @@ int mfx_vegas_refine(double* grid, const double* hist, int ndim, int nbins, doub
  * wrote them. */
 int mfx_hadronic_points(const double* dense, const int* slot, const double* x12, int64_t nev, int64_t npass,
                         int nexternal, double* x_out, double* q2_out, void* stream);
+
+/* ------------------------------------------------ learned proposal (flow) */
+/* Hit-or-miss unweighting of nev weighted events (replaces handing them to MadGraph's
+ * lhe_parser unweight, lhe_writer.py:319-356): keep event e with probability
+ * min(1, w[e] / wmax), the uniform taken from the Philox stream (ev0 + e, 0xffffffff,
+ * iteration) with key (seed, 0x6d66).  keep (nev,) u8 device; index_out (nev,) i32 device
+ * receives the kept event indices in order; *nkeep_host (optional, synchronises) their
+ * number.  Events with w > wmax are kept with weight w / wmax, the others with weight 1. */
 int64_t mfx_unweight_workspace_size(int64_t nev);
 int mfx_unweight(const double* w, int64_t nev, double wmax, uint32_t seed, uint32_t iteration, uint64_t ev0,
                  uint8_t* keep, int* index_out, void* workspace, int64_t workspace_bytes, int64_t* nkeep_host,
