@@ -44,12 +44,14 @@ PEAK_TFLOPS = {32: 157.3, 64: 78.6}   # MI355X published vector peaks (FP32 pack
 # passes scaled by a 1 GiB copy (profiles/pmc_k_smatrix_gg_ttxgg_f32.md for the fused
 # Feynman-diagram kernel, profiles/pmc_k_ordered_gg_ttxgg_f32.md for the colour-ordered
 # kernels, jamps staged through HBM included; 1 GiB copy calibration)
-HBM_BYTES_PER_ME = {("gg_ttxgg_fused", 32): 28180.3, ("gg_ttxgg", 32): 24776.7}
+HBM_BYTES_PER_ME = {("gg_ttxgg_fused", 32): 28180.3, ("gg_ttxgg", 32): 27656.8}
 # VALU wave instructions issued per ME (SQ_INSTS_VALU summed over the call's kernels / MEs,
-# same profiles): the executed-work side of the roofline.  A wave64 VALU instruction holds
-# a 16-lane SIMD for 4 cycles; 4 SIMDs per CU at the 2.4 GHz peak engine clock.
-VALU_WAVE_INSTS_PER_ME = {("gg_ttxgg", 32): 18802.7}
-VALU_CYCLES_PER_INST = 4
+# same profiles): the executed-work side of the roofline.  The published FP32 peak is 32 lanes
+# of a SIMD a cycle (157.3 TFLOP/s = 256 CUs x 4 SIMDs x 32 lanes x 2 x 2.4 GHz), so a wave64
+# FP32 instruction holds its SIMD for 2 cycles at that peak.  One wave issues at most one
+# instruction in 4 cycles; with two on a SIMD the kernels were measured at 1.35 in 4 cycles.
+VALU_WAVE_INSTS_PER_ME = {("gg_ttxgg", 32): 18997.4}
+VALU_CYCLES_PER_INST = 2
 ENGINE_HZ = 2.4e9
 METRIC = "unweighted events/sec at sigma/sigma=1e-3 and ME evals/sec, gg->ttgg on 1 MI355X"
 
