@@ -462,6 +462,10 @@ struct ProcessEntry {
 // events (about half a group's time), and a CU takes one such block at a time for the
 // purpose of this estimate, so a smaller E is faster until the blocks outnumber the CUs:
 // u u~ > t t~ g g FP64, 1,000 events: E = 64 259 us, 16 37 us; 30,001 events: 64 522 us, 16 526 us.
+// Of equal costs the smallest E whose rows still fill a block is taken, as several blocks on a CU
+// overlap: 10,000 events, E = 64 and 16, t t~ g FP32 41.0 and 31.6 us, FP64 46.5 and 37.6 us,
+// u u~ > t t~ g g FP64 193 and 149 us; 20,000 events, E = 32 and 16, 53.6 and 49.5, 69.8 and 62.1,
+// 287 and 253 us.
 // With few groups of rows the FP32 load (the invariants in FP64) is no longer small beside
 // them, and k_smatrix, which loads an event once, is faster from 1,024 events a CU on:
 // u u~ > t t~ g FP32 200,000 events 110 us against 102 us, 1e6 events 400 us against 475 us.
@@ -479,7 +483,7 @@ int events_per_block(int64_t nev) {
   for (int E = 64; E >= 4; E /= 2) {
     const int64_t blocks = (nev + E - 1) / E;
     const int64_t cost = (blocks + cus - 1) / cus * (2 * ((groups * E + 255) / 256) + 1);
-    if (cost < least) {
+    if (cost < least || (cost == least && groups * E >= 256)) {
       least = cost;
       best = E;
     }
