@@ -25,7 +25,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .vegas import MEIntegrand, _merge, _ptr, ALPHA, PROCESS_SETUP
+from .vegas import MEIntegrand, _merge, _ptr, with_luminosity, ALPHA, PROCESS_SETUP
 
 
 class McChannel(ctypes.Structure):
@@ -266,7 +266,7 @@ class MultiChannelIntegrand(MEIntegrand):
             # couplings at each event's scale, and the parton luminosity folded into the
             # matrix elements of the passing events (compact order)
             params, lumi = self._hadronic_factors(b, n, npass)
-            me = self._smatrix_timed(b, npass, params) * lumi
+            me = with_luminosity(self._smatrix_timed(b, npass, params), lumi)
         else:
             me = self._smatrix_timed(b, npass)
         _lib.check(self.lib.mfx_vegas_accumulate(

@@ -295,7 +295,7 @@ class MEIntegrand:
         if self.hadronic and npass:
             # f = luminosity x |M|^2 x weight (madflow_exec.py:455-459); the accumulation
             # multiplies the weights of the passing events
-            me = me * lumi
+            me = with_luminosity(me, lumi)
         _lib.check(self.lib.mfx_vegas_accumulate(
             ctypes.byref(self.p), ev0, n, iteration, _ptr(y_in), _ptr(b["slot"]), _ptr(me), _ptr(b["wps"]),
             None, _ptr(b["f"]) if keep_f else None, _ptr(b["ws"]), b["ws"].numel(), _ptr(b["result"]), s))
@@ -445,6 +445,19 @@ class MEIntegrand:
         var = max((tot[1] / N - mean * mean) / (N - 1.0), 0.0)
         return dict(I=mean, var=var, sigma=math.sqrt(var), wmax=tot[2], nonzero=tot[3], npass=npass, n=n_events,
                     sum_f=tot[0])
+
+
+def with_luminosity(me, lumi):
+    """Matrix elements times parton luminosities, one real value an event.  The library reads the
+    products by address, so what a density of another shape or type than the events' would
+    make of them (a column of n values: n x n products) is refused here; one value for all
+    events, or a row of n, is taken."""
+    f = me * lumi
+    if f.dtype != me.dtype:
+        raise TypeError("the parton luminosity must be real, got %s" % lumi.dtype)
+    if f.numel() != me.numel():
+        raise ValueError("the parton luminosity has shape %s for %d events" % (tuple(lumi.shape), me.numel()))
+    return f.reshape(-1)
 
 
 def _merge(a, b):
