@@ -798,7 +798,10 @@ __global__ void __launch_bounds__(GEN_BLOCK) k_hadronic_points(const double* __r
   if (!q2_out) return;
   const double* d = dense + (int64_t)s * nexternal * 4;
   double mt = 0.0;
-  for (int l = 2; l < nexternal; ++l) mt += sqrt(fmax(square_difference(d[4 * l], d[4 * l + 3]), 0.0));
+  for (int l = 2; l < nexternal; ++l) {
+    const double mt2 = square_difference(d[4 * l], d[4 * l + 3]);
+    mt += sqrt(mt2 < 0.0 ? 0.0 : mt2);     // not fmax, which would make 0 of an undefined mass
+  }
   q2_out[s] = 0.25 * mt * mt;
 }
 

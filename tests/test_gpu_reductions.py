@@ -172,3 +172,25 @@ def test_generation_by_number_of_legs(dev, n_out, massive):
     cut, _, _, _, idx = gen(x)
     want = torch.nonzero(torch.hypot(ps[:, -1, 1], ps[:, -1, 2]) > 300.0)
     assert torch.equal(idx.long(), want) and torch.equal(cut, ps[want[:, 0]])
+
+
+@pytest.mark.gpu
+def test_hadronic_points_of_undefined_momenta(dev):
+    """The scale of an event whose transverse mass is not a number is not a number either, as
+    elementwise operations give it; negative squares count as zero."""
+    n = 8
+    dense = torch.ones((n, 5, 4), dtype=torch.float64)
+    dense[..., 0] = 3.0
+    dense[1, 2, 0], dense[2, 4, 3] = math.nan, math.nan
+    dense[3, 3, 0] = dense[3, 3, 3] = math.inf
+    dense[4, 3, 0] = math.inf
+    dense[5, 2, 0] = 0.5
+    x12 = torch.rand((n, 2), dtype=torch.float64)
+    d, x, s = dense.to(dev), x12.to(dev), torch.arange(n, dtype=torch.int32, device=dev)
+    x_out, q2 = torch.empty((2, n), dtype=torch.float64, device=dev), torch.empty(n, dtype=torch.float64, device=dev)
+    ig = MEIntegrand("gg_ttxg", 13000.0, mapping="hadronic", pdf=lambda x, q2: x)
+    _lib.check(ig.lib.mfx_hadronic_points(_ptr(d), _ptr(s), _ptr(x), n, n, 5, _ptr(x_out), _ptr(q2), _lib.stream_ptr(dev)))
+    out = dense[:, 2:]
+    want = (0.5 * torch.sqrt(torch.clamp(out[..., 0] ** 2 - out[..., 3] ** 2, min=0.0)).sum(1)) ** 2
+    assert bool(torch.isnan(want[1:4]).all())
+    torch.testing.assert_close(q2.cpu(), want, rtol=1e-15, atol=0.0, equal_nan=True)
