@@ -704,9 +704,16 @@ __global__ void __launch_bounds__(BLOCK) k_ordered_mirror(OrderedArgs a) {
 #pragma unroll
           for (int q = 2; q < 6; ++q) J[x][y][q] = J[x + 1][y + 1][q];
           SD[x][y] = SD[x + 1][y + 1];
-          // momenta are added up again rather than carried in registers
-          J[x][y][0] = J[x][y - 1][0] + J[y][y][0];
-          J[x][y][1] = J[x][y - 1][1] + J[y][y][1];
+        }
+      }
+      // momenta are added up again rather than carried in registers, in ordered_ranges' order: a
+      // word's bits do not depend on the word its block began with
+#pragma unroll
+      for (int y = 1; y < NG - 1; ++y) {
+#pragma unroll
+        for (int x = y - 1; x >= 0; --x) {
+          J[x][y][0] = J[x][x][0] + J[x + 1][y][0];
+          J[x][y][1] = J[x][x][1] + J[x + 1][y][1];
         }
       }
       J[NG - 1][NG - 1] = first;
