@@ -767,10 +767,12 @@ template <> struct Vec4<double> { typedef mfx_f64x4 type; };
 // every k-step s), then each lane dots its D entries with jamps it already holds.  For
 // that, the colour of A row drow(q, r) of row tile mt is 4 (4 mt + r) + q: the output the
 // lane holds in register r is then the row of the colour of its k-step 4 mt + r, and the
-// jamps are read once.  The four lane quarters of each event are summed at the end.
+// jamps are read once.  The four lane quarters of each event are summed at the end of a row.
+// The rows are added in pairs, the pairs in pairs, and so on (their number is a power of two).
 // With more than one range of rows (few events: the rows of one tile are then spread over
-// the chip) a wave leaves its 16 sums in place of jamps that it alone has read, colour 0 of
-// its first row, and k_colour_sum adds the ranges in order.
+// the chip) a wave leaves its 16 sums of a range, a whole branch of that tree each, in place of
+// jamps that it alone has read, colour 0 of the range's first row, and k_colour_sum adds the
+// branches: an event's bits do not depend on the split, and so not on the size of the call.
 template <class T, class R>
 __global__ void __launch_bounds__(256) k_colour_mfma(void* jbuf, int64_t n, int64_t ld, int nhel, int hper,
                                                      double scale, int accumulate, double* out) {
@@ -778,10 +780,15 @@ __global__ void __launch_bounds__(256) k_colour_mfma(void* jbuf, int64_t n, int6
   constexpr int NCP = (NC + 15) / 16 * 16;    // padded colour rows of D
   constexpr int KS = NC / 4;                  // k-steps (NCOLOR is a multiple of 4)
   static_assert(NC % 4 == 0, "NCOLOR must be a multiple of 4");
+  constexpr int LEVELS = T::NCOMB <= 64 ? 6 : 7;
+  static_assert(T::NCOMB <= 1 << LEVELS, "one branch in wait for each level of the tree");
   typedef typename Vec4<R>::type V4;
   // integer numerators, rows permuted as above: exact in float.  Four columns per load and every
   // load in flight at once: with 120 colours the block reads 61 KB before it starts.
   __shared__ __attribute__((aligned(16))) float cf[NCP * NC];
+  // the branches in wait for their right-hand neighbours (12 registers would cost t t~ g g in FP32 two
+  // of eight waves a SIMD: 100,000 events 300 us instead of 282)
+  __shared__ double branch[LEVELS][4][16];
 #pragma unroll
   for (int i0 = 0; i0 < NCP * NC / 4; i0 += 256) {
     const int i = i0 + threadIdx.x;
@@ -837,11 +844,14 @@ __global__ void __launch_bounds__(256) k_colour_mfma(void* jbuf, int64_t n, int6
         // accumulators at once
         __builtin_amdgcn_sched_barrier(0);
       }
-      acc += double(part);
+      // sum the four lane quarters that hold the colours of each event
+      acc = double(part);
+      acc += __shfl_xor(acc, 16, 64);
+      acc += __shfl_xor(acc, 32, 64);
+      int up = 0;
+      for (int k = h - h0; k & 1; k >>= 1) acc += branch[up++][wave][lr];
+      if (h + 1 < h1) branch[up][wave][lr] = acc;
     }
-    // sum the four lane quarters that hold the colours of each event
-    acc += __shfl_xor(acc, 16, 64);
-    acc += __shfl_xor(acc, 32, 64);
     if (lq == 0 && ea < n) {
       if (parts > 1) reinterpret_cast<double*>(static_cast<cx<R>*>(jbuf) + (int64_t)h0 * NC * ld + tile * 16)[lr] = acc;
       else out[ea] = (accumulate ? out[ea] : 0.0) + acc * scale;
@@ -849,21 +859,31 @@ __global__ void __launch_bounds__(256) k_colour_mfma(void* jbuf, int64_t n, int6
   }
 }
 
-// the row ranges' sums of k_colour_mfma; step: jamps (complex R) from one range's first row to the
-// next one's.  16 events a block, 16 lanes an event: each adds every 16th range, then the
-// lanes are added in a fixed tree.  (One lane an event walking 64 ranges took 17 us, now 3.9 us.)
+// The branches of k_colour_mfma, parts (a power of two up to 128) an event; step: jamps (complex R)
+// from one range's first row to the next one's.  16 events a block, 16 lanes an event: each adds
+// the branch of its neighbouring ranges, then the lanes are added as the tree goes on.
+// (One lane an event walking 64 ranges took 17 us, now 3.9 us.)
 template <class R>
 __global__ void __launch_bounds__(256) k_colour_sum(const void* jbuf, int64_t n, int64_t step, int parts, double scale,
                                                     int accumulate, double* out) {
-  const int lane = threadIdx.x & 15;
+  constexpr int U = 8;
+  const int lane = threadIdx.x & 15, per = parts < 16 ? 1 : parts / 16;
   const int64_t e = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  double acc = 0.0;
-  if (e < n) {
-    const cx<R>* J = static_cast<const cx<R>*>(jbuf) + e / 16 * 16;
-    for (int p = lane; p < parts; p += 16) acc += reinterpret_cast<const double*>(J + p * step)[e % 16];
+  double v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int p = lane * per + u;
+    v[u] = 0.0;
+    if (e < n && u < per && p < parts)
+      v[u] = reinterpret_cast<const double*>(static_cast<const cx<R>*>(jbuf) + e / 16 * 16 + p * step)[e % 16];
   }
 #pragma unroll
-  for (int off = 8; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  for (int w = 1; w < U; w *= 2)
+#pragma unroll
+    for (int u = 0; u < U; u += 2 * w) v[u] += v[u + w];
+  double acc = v[0];
+#pragma unroll
+  for (int off = 1; off < 16; off *= 2) acc += __shfl_xor(acc, off, 64);
   if (lane == 0 && e < n) out[e] = (accumulate ? out[e] : 0.0) + acc * scale;
 }
 
@@ -945,10 +965,12 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
       a.cparts = (count + a.cper - 1) / a.cper;
       a.cper *= unit;
       // The colour sum's waves take (tile, range of rows) items in turn, so that a block stages its
-      // matrix once: as many blocks as a CU holds (61 KB of matrix each at 120 colours: two).
+      // matrix once: as many blocks as a CU holds (61 KB of matrix each at 120 colours: two), in FP64
+      // fewer, as four already read at the rate of the memory (t t~ g g, 100,000 events: 489 us with
+      // four, 521 us with eight; 30,000: 169 and 182 us).
       // The rows are split until every wave has COLOUR_ITEMS items, so that few events fill the
       // chip and the last round of many is short.
-      const int64_t cslots = (int64_t)cus * (T::NCOLOR > 64 ? 2 : 8);
+      const int64_t cslots = (int64_t)cus * (T::NCOLOR > 64 ? 2 : precision == 64 ? 4 : 8);
       int hper = hg;
       while (hper > 1 && tiles * (hg / hper) < COLOUR_ITEMS * 4 * cslots) hper /= 2;
       const int hparts = (hg + hper - 1) / hper;

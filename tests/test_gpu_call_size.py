@@ -1,6 +1,6 @@
-"""A point's amplitudes do not depend on the size of the call it comes in: the launches of few
-events, whose colour orderings are spread over the chip, give the bits of a launch in which one
-block walks every ordering."""
+"""A point's amplitudes and matrix element do not depend on the size of the call it comes in:
+the launches of few events, whose colour orderings and helicity rows are spread over the chip,
+give the bits of a launch in which one block walks every ordering and every row."""
 
 import pytest
 import torch
@@ -31,3 +31,23 @@ def test_jamps_of_split_orderings(dev, name, precision):
         me_n, jamp_n = m._matrix(ps[:n], hel, _vals(m), return_jamp=True)
         assert torch.equal(jamp_n, jamp[:n])
         assert torch.equal(me_n, me[:n])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("name,large", [("gg_ttxgg", 600000), ("gg_ttxggg", 150000)])
+def test_matrix_elements_of_split_rows(dev, name, large, precision):
+    """large: enough events that no row range is split off (the colour sum of a tile's rows is one
+    wave's); the sizes split them into ranges of one row, of some, and of half of them."""
+    m, _ = load_matrix(name, precision=precision)
+    base = torch.from_numpy(phase_space_points(name, 4097, seed=42)[0]).to(dev)
+    m.workspace_limit = 48 << 30       # every row of every event in one pass
+    ref = m.smatrix(base.repeat(large // base.shape[0] + 1, 1, 1), *_vals(m))
+    assert torch.equal(ref[:4097], ref[4097:8194])
+    for n in (1, 16, 17, 64, 65, 1000, 4097):
+        print("rows", name, precision, n, flush=True)
+        assert torch.equal(m.smatrix(base[:n], *_vals(m)), ref[:n])
+    for n in (20000, 40000, 70000):
+        print("rows", name, precision, n, flush=True)
+        got = m.smatrix(base.repeat(n // base.shape[0] + 1, 1, 1), *_vals(m))
+        assert torch.equal(got[:4097], ref[:4097])
