@@ -233,6 +233,7 @@ __device__ __forceinline__ VslashF<R> word_top_line(W<R> (&O)[NG], const W<R> (&
 // its reversal.
 template <int NG, int NC>
 struct MirrorWalk {
+  static_assert(NC <= 256, "colour rows are bytes");
   unsigned char at[NC / 2], rev[NC / 2];
 };
 template <int NG, int NC>
@@ -981,7 +982,9 @@ hipError_t launch_ordered(const SmatrixArgs& s, int precision, int per_helicity,
       const int64_t step = (int64_t)hper * T::NCOLOR * a.ld;
       const dim3 gs((unsigned)tiles);
       if (precision == 32) {
-        if (T::NG > 4 || s.use_helv) hipLaunchKernelGGL((k_ordered_jamps<T, 64, true>), gj, dim3(64), 0, st, a);
+        // five gluons: the layout of both is the same, so one kernel takes both calls
+        if constexpr (T::NG > 4) hipLaunchKernelGGL((k_ordered_jamps<T, 64, true>), gj, dim3(64), 0, st, a);
+        else if (s.use_helv) hipLaunchKernelGGL((k_ordered_jamps<T, 64, true>), gj, dim3(64), 0, st, a);
         else hipLaunchKernelGGL((k_ordered_jamps<T, 64, false>), gj, dim3(64), 0, st, a);
         hipLaunchKernelGGL((k_colour_mfma<T, float>), gc, dim3(256), 0, st, ws, n, a.ld, hg, hper, scale, acc, s.out + off);
         if (hparts > 1)
