@@ -326,12 +326,11 @@ __global__ void __launch_bounds__(256) k_smatrix(SmatrixArgs a) {
   }
 }
 
-// Rows evaluated two at a time by amplitudes2 in k_smatrix_rows, both precisions: the shared
-// currents are a quarter to a half of a row's work.  1e6 events FP64, one row at a time -> two:
-// t t~ 585 -> 352 us, t t~ g 4.52 -> 3.86 ms, u u~ > t t~ 189 -> 126 us, u u~ > t t~ g 968 -> 695 us,
-// u u~ > t t~ g g 15.8 -> 14.0 ms (although it spills 636 B a lane instead of 196).
-template <class T> struct PairedRows {
-  static constexpr bool value = T::MULTI_K == 1;
+// The processes that k_smatrix_rows takes: rows in pairs, a lane for each pair of an event, and
+// fewer than 24 colour flows (whose colour sum needs every lane of a wave at once, or whose
+// rows fill the register file by themselves).
+template <class T, class R> struct SideBySide {
+  static constexpr bool value = T::MULTI_K == 1 && T::NCOMB <= 128 && T::NCOLOR < 24 && !MfmaColour<T, R>::value;
 };
 
 // Waves per SIMD that k_smatrix_rows is compiled for: two where 256 registers hold a pair of
@@ -342,8 +341,11 @@ template <class T, class R> struct RowsWaves {
   static constexpr int value = T::NCOLOR <= (StableForms<R>::value ? 6 : 4) ? 2 : 1;
 };
 
-// The helicity rows of an event side by side: a block takes E events (a power of two up to 64)
-// and spreads their rows, or pairs of rows, over its 256 lanes, 256 / E at a time.  Each
+// The helicity rows of an event side by side, for processes whose rows come in pairs
+// (amplitudes2; the currents two rows share are a quarter to a half of a row's work: 1e6
+// events FP64, one row at a time -> two: t t~ 585 -> 352 us, t t~ g 4.52 -> 3.86 ms, u u~ > t t~ 189 ->
+// 126 us, u u~ > t t~ g 968 -> 695 us, u u~ > t t~ g g 15.8 -> 14.0 ms).  A block takes E events (a power of two
+// up to 64) and spreads their pairs of rows over its 256 lanes, 256 / E at a time.  Each
 // row's colour sum goes to LDS and one lane per event adds the rows in k_smatrix's order, so
 // the FP32 result is the same to the last bit.  A lane that walks every row by itself leaves
 // the chip idle for few events and ends larger calls in a half-empty round: per call, one lane
@@ -353,30 +355,22 @@ template <class T, class R> struct RowsWaves {
 template <class T, class R>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RowsWaves<T, R>::value)))
 k_smatrix_rows(SmatrixArgs a, int64_t ev0, int E) {
-  constexpr bool PAIR = PairedRows<T>::value;
-  constexpr int PER = PAIR ? 2 : 1, NGRP = T::NCOMB / PER;
-  static_assert(NGRP <= 64, "one lane per group of rows");
+  static_assert(SideBySide<T, R>::value, "one lane per pair of rows");
+  constexpr int NPAIR = T::NCOMB / 2;
   __shared__ R rows[T::NCOMB * 64];
-  __shared__ unsigned short group[64];
-  __shared__ int ngroup;
+  __shared__ unsigned short pair[64];
+  __shared__ int npair;
   const int t = threadIdx.x;
-  if (t < 64) {                          // the groups of rows that do not vanish, in order
-    unsigned hb = 0u;
-    if (t < NGRP) {
-      if constexpr (PAIR) {
-        constexpr int X = T::MULTI_LEG[0];
-        hb = ((unsigned)t & ((1u << X) - 1u)) | (((unsigned)t >> X) << (X + 1));
-      } else {
-        hb = T::hel_bits(t);
-      }
-    }
-    const bool live = t < NGRP && T::live(hb);
+  if (t < 64) {                          // the pairs of rows that do not vanish, in order
+    constexpr int X = T::MULTI_LEG[0];
+    const unsigned hb = t < NPAIR ? ((unsigned)t & ((1u << X) - 1u)) | (((unsigned)t >> X) << (X + 1)) : 0u;
+    const bool live = t < NPAIR && T::live(hb);
     const unsigned long long mask = __ballot(live);
-    if (live) group[__popcll(mask & ((1ull << t) - 1ull))] = (unsigned short)hb;
-    if (t == 0) ngroup = __popcll(mask);
+    if (live) pair[__popcll(mask & ((1ull << t) - 1ull))] = (unsigned short)hb;
+    if (t == 0) npair = __popcll(mask);
   }
   __syncthreads();
-  const int ng = ngroup, le = t & (E - 1);
+  const int np = npair, le = t & (E - 1);
   const int64_t e0 = ev0 + (int64_t)blockIdx.x * E + le;
   const int64_t e = e0 < a.nev ? e0 : a.nev - 1;
   R p[T::NEXTERNAL][4];
@@ -385,7 +379,7 @@ k_smatrix_rows(SmatrixArgs a, int64_t ev0, int E) {
   if constexpr (StableForms<R>::value) load_invariants<T, R>(a.all_ps, e, inv);
   const Params<R> prm = load_params<R>(a, e);
 #pragma unroll 1
-  for (int i = t / E; i < ng; i += 256 / E) {
+  for (int i = t / E; i < np; i += 256 / E) {
 #pragma unroll
     for (int l = 0; l < T::NEXTERNAL; ++l)
 #pragma unroll
@@ -394,22 +388,15 @@ k_smatrix_rows(SmatrixArgs a, int64_t ev0, int E) {
 #pragma unroll
       for (int k = 0; k < T::NINV; ++k) opaque(inv[k]);
     }
-    const unsigned hb = group[i];
-    cx<R> jamp[T::NCOLOR];
-    if constexpr (PAIR) {
-      cx<R> jamp2[T::NCOLOR];
-      T::template amplitudes2<R>(p, inv, hb, prm, jamp, jamp2);
-      rows[2 * i * E + le] = colour_numerator<T, R>(jamp);
-      rows[(2 * i + 1) * E + le] = colour_numerator<T, R>(jamp2);
-    } else {
-      T::template amplitudes<R>(p, inv, hb, nullptr, prm, jamp);
-      rows[i * E + le] = colour_numerator<T, R>(jamp);
-    }
+    cx<R> jamp[T::NCOLOR], jamp2[T::NCOLOR];
+    T::template amplitudes2<R>(p, inv, pair[i], prm, jamp, jamp2);
+    rows[2 * i * E + le] = colour_numerator<T, R>(jamp);
+    rows[(2 * i + 1) * E + le] = colour_numerator<T, R>(jamp2);
   }
   __syncthreads();
   if (t < E && e0 < a.nev) {
     R ans = R(0);
-    for (int i = 0; i < PER * ng; ++i) ans += rows[i * E + t] * R(1.0 / T::CF_DEN);
+    for (int i = 0; i < 2 * np; ++i) ans += rows[i * E + t] * R(1.0 / T::CF_DEN);
     a.out[e0] = double(ans) / T::DENOMINATOR;
   }
 }
@@ -438,12 +425,11 @@ __global__ void __launch_bounds__(256) k_matrix_hel(SmatrixArgs a) {
   }
 }
 
-// Whether large calls run k_smatrix: the processes with 24 colour flows (whose colour sum needs
-// every lane of a wave at once, or whose rows fill the register file by themselves), and
-// FP32 with few groups of rows.
+// Whether large calls run k_smatrix: the processes that k_smatrix_rows does not take, and FP32 with
+// few pairs of rows.
 template <class T, class R> struct KeepsEvents {
   static constexpr bool value =
-      T::NCOLOR >= 24 || (StableForms<R>::value && T::NCOMB / (T::FILTERED ? 4 : 2) < 16);
+      !SideBySide<T, R>::value || (StableForms<R>::value && T::NCOMB / (T::FILTERED ? 4 : 2) < 16);
 };
 
 struct ProcessEntry {
@@ -458,21 +444,21 @@ struct ProcessEntry {
 };
 
 // Which kernel takes a call, and E: k_smatrix_rows (E > 0) or k_smatrix (0).
-// A block of k_smatrix_rows works through ceil(groups E / 256) groups of rows after loading its
-// events (about half a group's time), and a CU takes one such block at a time for the
+// A block of k_smatrix_rows works through ceil(pairs E / 256) pairs of rows after loading its
+// events (about half a pair's time), and a CU takes one such block at a time for the
 // purpose of this estimate, so a smaller E is faster until the blocks outnumber the CUs:
 // u u~ > t t~ g g FP64, 1,000 events: E = 64 259 us, 16 37 us; 30,001 events: 64 522 us, 16 526 us.
 // Of equal costs the smallest E whose rows still fill a block is taken, as several blocks on a CU
 // overlap: 10,000 events, E = 64 and 16, t t~ g FP32 41.0 and 31.6 us, FP64 46.5 and 37.6 us,
 // u u~ > t t~ g g FP64 193 and 149 us; 20,000 events, E = 32 and 16, 53.6 and 49.5, 69.8 and 62.1,
 // 287 and 253 us.
-// With few groups of rows the FP32 load (the invariants in FP64) is no longer small beside
+// With few pairs of rows the FP32 load (the invariants in FP64) is no longer small beside
 // them, and k_smatrix, which loads an event once, is faster from 1,024 events a CU on:
 // u u~ > t t~ g FP32 200,000 events 110 us against 102 us, 1e6 events 400 us against 475 us.
-// With 16 groups or more it is not (u u~ > t t~ g g 1e6 events 4,934 us against 4,858 us).
+// With 16 pairs or more it is not (u u~ > t t~ g g 1e6 events 4,934 us against 4,858 us).
 template <class T, class R>
 int events_per_block(int64_t nev) {
-  constexpr int groups = T::NCOMB / (PairedRows<T>::value ? 2 : 1) / (T::FILTERED ? 2 : 1);
+  constexpr int pairs = T::NCOMB / (T::FILTERED ? 4 : 2);
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
@@ -482,8 +468,8 @@ int events_per_block(int64_t nev) {
   int64_t least = INT64_MAX;
   for (int E = 64; E >= 4; E /= 2) {
     const int64_t blocks = (nev + E - 1) / E;
-    const int64_t cost = (blocks + cus - 1) / cus * (2 * ((groups * E + 255) / 256) + 1);
-    if (cost < least || (cost == least && groups * E >= 256)) {
+    const int64_t cost = (blocks + cus - 1) / cus * (2 * ((pairs * E + 255) / 256) + 1);
+    if (cost < least || (cost == least && pairs * E >= 256)) {
       least = cost;
       best = E;
     }
@@ -493,7 +479,7 @@ int events_per_block(int64_t nev) {
 
 template <class T, class R>
 hipError_t launch_smatrix(const SmatrixArgs& a, hipStream_t s) {
-  if constexpr (!MfmaColour<T, R>::value && T::NCOLOR < 24) {
+  if constexpr (SideBySide<T, R>::value) {
     const int E = events_per_block<T, R>(a.nev);
     if (E) {
       const int64_t most = (int64_t)E << 22;        // events of one launch (its threads fit 32 bits)
