@@ -68,13 +68,12 @@ struct KSum {
 template <int D = 0>
 __device__ __forceinline__ void uniforms(const GenConst& g, uint64_t ev, uint32_t iteration, double* y) {
   const int ndim = D ? D : g.ndim;
-#pragma clang loop unroll_count(D ? 32 : 1)
-  for (int j = 0; 2 * j < ndim; ++j) {
+  for_each<D != 0>((ndim + 1) / 2, [&](int j) {
     double u0, u1;
     philox_pair(ev, (uint32_t)j, g.seed, iteration, u0, u1);
     y[2 * j] = u0;
     if (2 * j + 1 < ndim) y[2 * j + 1] = u1;
-  }
+  });
 }
 
 // A coordinate of an external proposal, clamped into [0, 1] so that bin indices stay in range
@@ -89,11 +88,10 @@ template <int D = 0>
 __device__ __forceinline__ bool external_point(const float* __restrict__ src, int nd, double* y) {
   const int ndim = D ? D : nd;
   bool ok = true;
-#pragma clang loop unroll_count(D ? 32 : 1)
-  for (int d = 0; d < ndim; ++d) {
+  for_each<D != 0>(ndim, [&](int d) {
     ok = ok && isfinite(src[d]);
     y[d] = external_coord(src[d]);
-  }
+  });
   return ok;
 }
 
@@ -102,8 +100,7 @@ __device__ __forceinline__ double vmap(const GenConst& g, const double* __restri
                                        int* bins) {
   double jac = 1.0;
   const int nb = g.nbins, ndim = D ? D : g.ndim;
-#pragma clang loop unroll_count(D ? 32 : 1)
-  for (int d = 0; d < ndim; ++d) {
+  for_each<D != 0>(ndim, [&](int d) {
     const double xn = y[d] * nb;
     int b = (int)xn;
     if (b >= nb) b = nb - 1;
@@ -112,7 +109,7 @@ __device__ __forceinline__ double vmap(const GenConst& g, const double* __restri
     x[d] = lo + w * (xn - b);
     jac *= w * nb;
     if (bins) bins[d] = b;
-  }
+  });
   return jac;
 }
 
@@ -121,37 +118,45 @@ __device__ __forceinline__ double eta_of(const double* p) {
   return 0.5 * log((pa + p[3]) / (pa - p[3]));
 }
 
-// N: as in mfx_phasespace.h; every leg is then indexed by a constant and selected by its number
+// f(i) for the legs lo <= i <= hi until one is false.  N: as in mfx_phasespace.h; every leg is then
+// indexed by a constant and selected by its number.
+template <int N, class F> __device__ __forceinline__ bool every_leg(int lo, int hi, F&& f) {
+  if constexpr (N != 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (i >= lo && i <= hi && !f(i)) return false;
+  } else {
+    for (int i = lo; i <= hi; ++i)
+      if (!f(i)) return false;
+  }
+  return true;
+}
+
 template <int N = 0>
 __device__ __forceinline__ bool pass_cuts(const GenConst& g, double (*p)[4]) {
-  const int n = N ? N : g.rc.n;
-#pragma clang loop unroll_count(N ? 32 : 1)
-  for (int i = 0; i < n; ++i) {
-    if (i < g.cut_first || i > g.cut_last) continue;
-    const double pt = sqrt(p[i][1] * p[i][1] + p[i][2] * p[i][2]);
-    if (!(pt > g.pt_min)) return false;
-    if (g.abs_eta_max > 0.0 && !(fabs(eta_of(p[i])) < g.abs_eta_max)) return false;
-  }
-  if (g.dr_min > 0.0) {
-#pragma clang loop unroll_count(N ? 32 : 1)
-    for (int i = 0; i < n; ++i)
-#pragma clang loop unroll_count(N ? 32 : 1)
-      for (int j = i + 1; j < n; ++j) {
-        if (i < g.cut_first || j > g.cut_last) continue;
-        const double de = eta_of(p[i]) - eta_of(p[j]);
-        double dp = fabs(atan2(p[i][2], p[i][1]) - atan2(p[j][2], p[j][1]));
-        if (dp > MFX_PI) dp = 2.0 * MFX_PI - dp;
-        if (!(de * de + dp * dp > g.dr_min * g.dr_min)) return false;
-      }
-  }
+  if (!every_leg<N>(g.cut_first, g.cut_last, [&](int i) {
+        const double pt = sqrt(p[i][1] * p[i][1] + p[i][2] * p[i][2]);
+        return pt > g.pt_min && !(g.abs_eta_max > 0.0 && !(fabs(eta_of(p[i])) < g.abs_eta_max));
+      }))
+    return false;
+  if (g.dr_min > 0.0 && !every_leg<N>(g.cut_first, g.cut_last, [&](int i) {
+        return every_leg<N>(i + 1, g.cut_last, [&](int j) {
+          const double de = eta_of(p[i]) - eta_of(p[j]);
+          double dp = fabs(atan2(p[i][2], p[i][1]) - atan2(p[j][2], p[j][1]));
+          if (dp > MFX_PI) dp = 2.0 * MFX_PI - dp;
+          return de * de + dp * dp > g.dr_min * g.dr_min;
+        });
+      }))
+    return false;
   // register_cut's predicates (phasespace.py:457-466): strict bounds on pt, mt or mt2
   for (int c = 0; c < g.ncuts; ++c) {
     const mfx_cut& k = g.cuts[c];
     double q[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma clang loop unroll_count(N ? 32 : 1)
-    for (int i = 0; i < n; ++i)
-      if (i == k.particle)
-        for (int m = 0; m < 4; ++m) q[m] = p[i][m];
+    every_leg<N>(k.particle, k.particle, [&](int i) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) q[m] = p[i][m];
+      return true;
+    });
     const double pt2 = q[1] * q[1] + q[2] * q[2];
     double v;
     if (k.variable == 0) {
@@ -190,15 +195,14 @@ __global__ void __launch_bounds__(GEN_BLOCK) k_generate(GenConst g, const double
     if (x_in) {
       // the caller's FP64 points, used as they are (no VEGAS grid): a non-finite coordinate
       // rejects the event, the others are clamped to [0, 1]
-#pragma clang loop unroll_count(N ? 32 : 1)
-      for (int d = 0; d < ndim; ++d) {
+      for_each<N != 0>(ndim, [&](int d) {
         double v = x_in[e * ndim + d];
         if (!isfinite(v)) {
           y_ok = false;
           v = 0.0;
         }
         x[d] = v < 0.0 ? 0.0 : (v > 1.0 ? 1.0 : v);
-      }
+      });
     } else {
       if (y_in) {
         y_ok = external_point<D>(y_in + e * ndim, ndim, y);
@@ -232,18 +236,17 @@ __global__ void __launch_bounds__(GEN_BLOCK) k_generate(GenConst g, const double
     if (MAP == 2 && g.lab_frame) {
       // boost along z to the lab frame, rapidity -eta = (1/2) ln(x1 / x2) (phasespace.py:322-357)
       const double eta = -0.5 * log(x1 / x2), ch = cosh(eta), sh = sinh(eta);
-#pragma clang loop unroll_count(N ? 32 : 1)
-      for (int i = 0; i < nexternal; ++i) {
+      for_each<N != 0>(nexternal, [&](int i) {
         const double E = p[i][0], pz = p[i][3];
         p[i][0] = ch * E - sh * pz;
         p[i][3] = ch * pz - sh * E;
-      }
+      });
     }
     double* out = all_ps + e * (nexternal * 4);
-#pragma clang loop unroll_count(N ? 32 : 1)
-    for (int i = 0; i < nexternal; ++i)
-#pragma clang loop unroll_count(N ? 32 : 1)
+    for_each<N != 0>(nexternal, [&](int i) {
+#pragma unroll
       for (int k = 0; k < 4; ++k) out[4 * i + k] = p[i][k];
+    });
     if (x12) {
       x12[2 * e] = x1;
       x12[2 * e + 1] = x2;

@@ -28,6 +28,18 @@ struct RamboConst {
 // registers), 0 where it is rc.n.
 template <int N> __device__ __forceinline__ int legs_of(const RamboConst& rc) { return N ? N : rc.n; }
 
+// f(0) .. f(n - 1): unrolled where the number is known (FIXED, n folded to a constant), else a loop
+// that the compiler unrolls as it sees fit: kept rolled, the general kernels took up to 27%
+// longer (2e6 points of six legs on RAMBO 1.38 ms, so 1.07).
+template <bool FIXED, class F> __device__ __forceinline__ void for_each(int n, F&& f) {
+  if constexpr (FIXED) {
+#pragma clang loop unroll_count(32)
+    for (int i = 0; i < n; ++i) f(i);
+  } else {
+    for (int i = 0; i < n; ++i) f(i);
+  }
+}
+
 // Newton iterations allowed for the massive rescaling factor xi
 constexpr int NEWTON_MAX = 50;
 
@@ -42,8 +54,7 @@ __device__ __forceinline__ double rambo_event(const RamboConst& rc, const double
                                               double (*p)[4], bool& converged) {
   const int n = legs_of<N>(rc);
   double Q[4] = {0, 0, 0, 0};
-#pragma clang loop unroll_count(N ? 8 : 1)
-  for (int i = 0; i < n; ++i) {
+  for_each<N != 0>(n, [&](int i) {
     const double costh = 2.0 * x[4 * i] - 1.0;
     const double sinth = sqrt(1.0 - costh * costh);
     double sphi, cphi;
@@ -53,24 +64,23 @@ __device__ __forceinline__ double rambo_event(const RamboConst& rc, const double
     p[i][1] = e * sinth * sphi;
     p[i][2] = e * sinth * cphi;
     p[i][3] = e * costh;
-#pragma clang loop unroll_count(N ? 8 : 1)
+#pragma unroll
     for (int k = 0; k < 4; ++k) Q[k] += p[i][k];
-  }
+  });
   const double M = sqrt(Q[0] * Q[0] - (Q[1] * Q[1] + Q[2] * Q[2] + Q[3] * Q[3]));
   const double iM = 1.0 / M;
   const double xs = sqrts * iM;
   const double b1 = -Q[1] * iM, b2 = -Q[2] * iM, b3 = -Q[3] * iM;
   const double gamma = Q[0] * iM;
   const double a = 1.0 / (1.0 + gamma);
-#pragma clang loop unroll_count(N ? 8 : 1)
-  for (int i = 0; i < n; ++i) {
+  for_each<N != 0>(n, [&](int i) {
     const double bq = p[i][1] * b1 + p[i][2] * b2 + p[i][3] * b3;
     const double t = bq * a + p[i][0];
     p[i][0] = (p[i][0] * gamma + bq) * xs;
     p[i][1] = (p[i][1] + b1 * t) * xs;
     p[i][2] = (p[i][2] + b2 * t) * xs;
     p[i][3] = (p[i][3] + b3 * t) * xs;
-  }
+  });
   double logw = rc.logw0 + (2 * n - 4) * log(sqrts);
   converged = true;
   if (rc.massive) logw += massive_rescale<N>(rc, sqrts, p, converged);
@@ -92,13 +102,12 @@ __device__ __forceinline__ double massive_rescale(const RamboConst& rc, double s
     for (int it = 0; it < NEWTON_MAX; ++it) {
       const double x2 = xi * xi;
       double f0 = -sqrts, g0 = 0.0;
-#pragma clang loop unroll_count(N ? 8 : 1)
-      for (int i = 0; i < n; ++i) {
+      for_each<N != 0>(n, [&](int i) {
         const double E2 = p[i][0] * p[i][0];
         const double nE = sqrt(rc.masses[i] * rc.masses[i] + E2 * x2);
         f0 += nE;
         g0 += E2 / nE;
-      }
+      });
       if (fabs(f0) <= 1e-14 * sqrts) {
         converged = true;
         break;
@@ -107,8 +116,7 @@ __device__ __forceinline__ double massive_rescale(const RamboConst& rc, double s
     }
     const double x2 = xi * xi;
     double wt2 = 1.0, wt3 = 0.0;
-#pragma clang loop unroll_count(N ? 8 : 1)
-    for (int i = 0; i < n; ++i) {
+    for_each<N != 0>(n, [&](int i) {
       const double v = p[i][0] * xi;
       const double nE = sqrt(rc.masses[i] * rc.masses[i] + p[i][0] * p[i][0] * x2);
       wt2 *= v / nE;
@@ -117,7 +125,7 @@ __device__ __forceinline__ double massive_rescale(const RamboConst& rc, double s
       p[i][1] *= xi;
       p[i][2] *= xi;
       p[i][3] *= xi;
-    }
+    });
     logw += (2 * n - 3) * log(xi) + log(wt2 / wt3 * sqrts);
   }
   return logw;
@@ -152,8 +160,7 @@ __device__ __forceinline__ double diet_event(const RamboConst& rc, const double*
   const int n = legs_of<N>(rc);
   double Q[4] = {sqrts, 0.0, 0.0, 0.0};
   double M = sqrts;
-#pragma clang loop unroll_count(N ? 8 : 1)
-  for (int i = 0; i < n - 1; ++i) {
+  for_each<N != 0>(n - 1, [&](int i) {
     double Mn = 0.0;
     if (i < n - 2) Mn = M * sqrt(diet_solve(x[i], n - 2 - i));
     const double q = (M * M - Mn * Mn) / (2.0 * M);
@@ -170,11 +177,11 @@ __device__ __forceinline__ double diet_event(const RamboConst& rc, const double*
     p[i][1] = k1 + b1 * c;
     p[i][2] = k2 + b2 * c;
     p[i][3] = k3 + b3 * c;
-#pragma clang loop unroll_count(N ? 8 : 1)
+#pragma unroll
     for (int j = 0; j < 4; ++j) Q[j] -= p[i][j];
     M = Mn;
-  }
-#pragma clang loop unroll_count(N ? 8 : 1)
+  });
+#pragma unroll
   for (int j = 0; j < 4; ++j) p[n - 1][j] = Q[j];
   double logw = rc.logw0 + (2 * n - 4) * log(sqrts);
   converged = true;
