@@ -225,9 +225,9 @@ template <class T> struct ColourLds<T, true> {
   float red[4][64];
 };
 
-// All helicity rows for nev events, an event's rows one after another on one lane.  The event loop is block-uniform so that
-// every lane of a wave reaches the wave-wide colour contraction; lanes past the end
-// evaluate the last event again and write nothing.
+// All helicity rows for nev events, an event's rows one after another on one lane.  The event
+// loop is block-uniform so that every lane of a wave reaches the wave-wide colour contraction;
+// lanes past the end evaluate the last event again and write nothing.
 template <class T, class R>
 __global__ void __launch_bounds__(256) k_smatrix(SmatrixArgs a) {
   constexpr bool MFMA = MfmaColour<T, R>::value;
@@ -425,11 +425,15 @@ __global__ void __launch_bounds__(256) k_matrix_hel(SmatrixArgs a) {
   }
 }
 
-// Whether large calls run k_smatrix: the processes that k_smatrix_rows does not take, and FP32 with
-// few pairs of rows.
+// Whether k_smatrix is built: for the processes that k_smatrix_rows does not take, and for FP32 with
+// few pairs of rows or one wave a SIMD, where its full rounds of 256 events a CU are the faster form:
+// from `fewest` of them on, if the last leaves less than 1 / slack of the others empty.
 template <class T, class R> struct KeepsEvents {
+  static constexpr int pairs = T::NCOMB / (T::FILTERED ? 4 : 2);
   static constexpr bool value =
-      !SideBySide<T, R>::value || (StableForms<R>::value && T::NCOMB / (T::FILTERED ? 4 : 2) < 16);
+      !SideBySide<T, R>::value || (StableForms<R>::value && (pairs < 16 || RowsWaves<T, R>::value == 1));
+  static constexpr int fewest = pairs >= 16 ? 1 : (T::NCOLOR > 2 ? 2 : 3);
+  static constexpr int slack = pairs >= 16 ? 40 : (T::NCOLOR > 2 ? 10 : 20);
 };
 
 struct ProcessEntry {
@@ -453,17 +457,28 @@ struct ProcessEntry {
 // u u~ > t t~ g g FP64 193 and 149 us; 20,000 events, E = 32 and 16, 53.6 and 49.5, 69.8 and 62.1,
 // 287 and 253 us.
 // With few pairs of rows the FP32 load (the invariants in FP64) is no longer small beside
-// them, and k_smatrix, which loads an event once, is faster from 1,024 events a CU on:
-// u u~ > t t~ g FP32 200,000 events 110 us against 102 us, 1e6 events 400 us against 475 us.
-// With 16 pairs or more it is not (u u~ > t t~ g g 1e6 events 4,934 us against 4,858 us).
+// them, and k_smatrix loads an event once, but its last round takes as long as a full one.  So it
+// is taken where that is full enough, and with more than four rounds always.  Rows side by side
+// and k_smatrix, us: t t~ 131,072 events 38.0 and 39.0, 196,608 55.0 and 54.0, 240,000 67.3 and 69.4, 262,144
+// 72.2 and 69.5, 1e6 262 and 252; u u~ > t t~ 131,072 14.5 and 14.7, 262,144 25.1 and 24.2, 1e6 85 and 79;
+// u u~ > t t~ g 100,000 56 and 61, 120,000 63.7 and 60.9, 196,608 94.5 and 84.6, 225,000 109.7 and 110.6, 262,144
+// 125 and 111, 1e6 473 and 398; u g > t t~ u 100,000 57 and 63, 120,000 64.7 and 62.6, 262,144 127 and 117.
+// With 16 pairs at one wave a SIMD (u u~ > t t~ g g) k_smatrix takes 2% less for an event: 65,536 events 316
+// and 311, 400,000 1,970 and 2,170, 983,040 4,720 and 4,630, 1e6 4,880 and 4,940, 3e6 14,500 and 14,200.
+// At two waves (t t~ g) it takes longer (1e6 events 1,840 and 2,340).
 template <class T, class R>
 int events_per_block(int64_t nev) {
-  constexpr int pairs = T::NCOMB / (T::FILTERED ? 4 : 2);
+  constexpr int pairs = KeepsEvents<T, R>::pairs;
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
     cus = 256;
-  if (KeepsEvents<T, R>::value && nev > 1024ll * cus) return 0;
+  if constexpr (KeepsEvents<T, R>::value) {
+    constexpr int fewest = KeepsEvents<T, R>::fewest, slack = KeepsEvents<T, R>::slack;
+    const int64_t round = 256ll * cus, rounds = (nev + round - 1) / round;
+    if (pairs < 16 && rounds > 4) return 0;
+    if (rounds >= fewest && slack * (rounds * round - nev) <= nev) return 0;
+  }
   int best = 64;
   int64_t least = INT64_MAX;
   for (int E = 64; E >= 4; E /= 2) {

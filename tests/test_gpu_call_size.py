@@ -51,3 +51,20 @@ def test_matrix_elements_of_split_rows(dev, name, large, precision):
         print("rows", name, precision, n, flush=True)
         got = m.smatrix(base.repeat(n // base.shape[0] + 1, 1, 1), *_vals(m))
         assert torch.equal(got[:4097], ref[:4097])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,sizes", [("uux_ttxgg", (63000, 65000, 65536, 65537, 131072)),
+                                        ("uux_ttxg", (110000, 120000, 131073, 240000, 262145)),
+                                        ("ug_ttxu", (119000, 119200, 131073)),
+                                        ("gg_ttx", (131072, 187000, 188000, 196609))])
+def test_rows_side_by_side_or_in_turn(dev, name, sizes):
+    """FP32 on both sides of the sizes (on 256 CUs) at which an event's rows go in turn on one lane."""
+    m, _ = load_matrix(name, precision=32)
+    base = torch.from_numpy(phase_space_points(name, 4097, seed=43)[0]).to(dev)
+    ps = base.repeat(max(sizes) // base.shape[0] + 1, 1, 1)
+    ref = m.smatrix(base, *_vals(m))
+    for n in sizes:
+        print("in turn", name, n, flush=True)
+        got = m.smatrix(ps[:n], *_vals(m))
+        assert torch.equal(got, ref.repeat(n // base.shape[0] + 1)[:n])
