@@ -302,22 +302,26 @@ struct OrderedStage {
   // 26.8 ms; spinors in private memory 28.7 ms, and three waves a SIMD with them 29.8 ms (272 B of
   // spills).  t t~ g g g, 50,000 events: one wave a SIMD 33.7 ms, two with 120 slots (5 waves a CU)
   // 32.2 ms, with 80 slots 26.6 ms although 224 B spill.
-  static constexpr bool COMPACT = !EXPLICIT && NG <= 4;
+  // An explicit helicity vector has one row, so one helicity of each fermion (SINGLE): 78 slots
+  // (131,072 events, one row: 102 slots 304 us, 78 slots 199 us); five gluons take both calls with
+  // the same layout.
+  static constexpr bool COMPACT = !EXPLICIT && NG <= 4, SINGLE = EXPLICIT && NG <= 4;
   static constexpr int GW = COMPACT ? 9 : 12;
   static constexpr int NWF = NG * GW;
   // the pair invariants gluon-gluon and top-gluon (pair_index), then anti-top-gluon
   static constexpr int NPI = (NG + 1) * NG / 2, NINV = NPI + NG;
   // the spinor components of the top and the anti-top at both helicities, staged once per event
   static constexpr int FB = NWF + NINV;
-  static constexpr int NFM = COMPACT ? 0 : 4;       // momentum slots of a fermion
-  static constexpr int NFS = COMPACT ? 30 : 40;
   static constexpr bool PRIVATE = NG > 4;           // the spinors in private memory
+  static constexpr int NFM = PRIVATE ? 4 : 0;       // momentum slots of a fermion
+  static constexpr int NFS = PRIVATE ? 40 : (SINGLE ? 16 : 30);
   static constexpr int NSLOT = NWF + NINV + (PRIVATE ? 0 : NFS);
+  static_assert(NSLOT <= 80, "eight waves a CU");
   // slot of component q (its real part; the imaginary part follows) of the top (anti = 0) or
   // the anti-top at helicity bit h
   static constexpr __device__ int fermion(int anti, int h, int q) {
-    return FB + (q < 2 ? 4 * anti + 2 * q
-                       : 2 * NFM + 16 * anti + (COMPACT && anti ? 7 : 8) * h + 2 * (q - 2));
+    if (SINGLE) return FB + 8 * anti + 2 * (q - 2);
+    return FB + (q < 2 ? 4 * anti + 2 * q : 2 * NFM + 16 * anti + (COMPACT && anti ? 7 : 8) * h + 2 * (q - 2));
   }
   // slot of component q (0, 1: momentum; 2..5: polarisation), part 0 / 1, of a gluon; -1: zero
   static constexpr __device__ int gluon(int q, int part) {
@@ -378,7 +382,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
   {
     const int* hv = EXPLICIT && a.s.use_helv ? a.s.helv : nullptr;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < (S::SINGLE ? 1 : 2); ++h) {
       W<R> top, atop;
       T::template fermions<R>(p, ((unsigned)h << T::TOP_LEG) | ((unsigned)h << T::ATOP_LEG), hv, prm, top, atop);
 #pragma unroll
@@ -391,7 +395,7 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
             spinor[oa - S::FB] = atop[q].re;
             spinor[oa + 1 - S::FB] = atop[q].im;
           }
-        } else if (q >= 2 || (h == 0 && !S::COMPACT)) {
+        } else if (q >= 2) {
           lds[ot * BLOCK + t] = top[q].re;
           lds[(ot + 1) * BLOCK + t] = top[q].im;
           lds[oa * BLOCK + t] = atop[q].re;
@@ -401,10 +405,17 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
       atop_last[h] = atop[5].im;
     }
   }
-  // spinor of the top (anti = 0) or anti-top (anti = 1) at helicity bit h, from LDS; COMPACT: the
-  // top's momentum slots from p, the anti-top's, which are not read, left out
+  // spinor of the top (anti = 0) or anti-top (anti = 1) at helicity bit h; from LDS with the top's
+  // momentum slots from p, the anti-top's, which are not read, left out
   auto staged_fermion = [&](int anti, int h, W<R>& w) {
-    if constexpr (S::COMPACT) {
+    if constexpr (S::PRIVATE) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        const int o = S::fermion(anti, h, q) - S::FB;
+        w[q].re = spinor[o];
+        w[q].im = spinor[o + 1];
+      }
+    } else {
       if (!anti) {
         w[0] = cx<R>(p[T::TOP_LEG][0], p[T::TOP_LEG][3]);
         w[1] = cx<R>(p[T::TOP_LEG][1], p[T::TOP_LEG][2]);
@@ -413,23 +424,11 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
       for (int q = 2; q < 6; ++q) {
         const int o = S::fermion(anti, h, q);
         w[q].re = lds[o * BLOCK + t];
-        if (q < 5 || !anti) {
+        if (!S::COMPACT || q < 5 || !anti) {
           w[q].im = lds[(o + 1) * BLOCK + t];
         } else {
           w[q].im = h ? atop_last[1] : atop_last[0];
           opaque(w[q].im);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) {
-        const int o = S::fermion(anti, h, q);
-        if constexpr (S::PRIVATE) {
-          w[q].re = spinor[o - S::FB];
-          w[q].im = spinor[o + 1 - S::FB];
-        } else {
-          w[q].re = lds[o * BLOCK + t];
-          w[q].im = lds[(o + 1) * BLOCK + t];
         }
       }
     }
@@ -611,14 +610,17 @@ __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2)))
 // -> 42.0 ms (its currents do not fit 512 registers: 1.4 KB of spills a lane).  Momenta of ranges
 // are added up again for each word; carried along they made t t~ g g spill and take 1,152 us.
 // LDS: the gluons, then the spinor components of the top and the anti-top at both helicities;
-// one wave per SIMD (the currents fill the registers), so four blocks a CU may take 40 KB each.
+// one wave per SIMD (the currents fill the registers), so four blocks a CU may take 40 KB each
+// (t t~ g g g, 131,072 events of one explicit row: 46 KB and three blocks 5.85 ms, 38 KB 4.60 ms).
 template <class T, bool EXPLICIT>
 struct MirrorStage {
   static constexpr int NG = T::NG;
   // a polarisation's time component and the imaginary part of its z component are zero, except
   // with an explicit helicity vector (BRST)
   static constexpr int GW = EXPLICIT ? 12 : 9;
-  static constexpr int FB = NG * GW, NSLOT = FB + 32;
+  // one row, so one helicity of each fermion, with an explicit vector
+  static constexpr int FB = NG * GW, NH = EXPLICIT ? 1 : 2, NSLOT = FB + 16 * NH;
+  static_assert(NSLOT * 64 * 8 <= 40 * 1024, "four blocks a CU");
   static constexpr __device__ int gluon(int q, int part) {
     if (EXPLICIT || q < 2) return 2 * q + part;
     return q == 2 ? -1 : (q == 5 ? (part ? -1 : 8) : 4 + 2 * (q - 3) + part);
@@ -656,23 +658,23 @@ __global__ void __launch_bounds__(BLOCK) k_ordered_mirror(OrderedArgs a) {
     }
   }
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < S::NH; ++h) {
     W<R> top, atop;
     T::template fermions<R>(p, ((unsigned)h << T::TOP_LEG) | ((unsigned)h << T::ATOP_LEG), helv, prm, top, atop);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int o = S::FB + 8 * h + 2 * q;
+      const int o = S::FB + 8 * h + 2 * q, oa = o + 8 * S::NH;
       lds[o * BLOCK + t] = top[q + 2].re;
       lds[(o + 1) * BLOCK + t] = top[q + 2].im;
-      lds[(o + 16) * BLOCK + t] = atop[q + 2].re;
-      lds[(o + 17) * BLOCK + t] = atop[q + 2].im;
+      lds[oa * BLOCK + t] = atop[q + 2].re;
+      lds[(oa + 1) * BLOCK + t] = atop[q + 2].im;
     }
   }
   // spinor components of the top (anti = 0) or anti-top (anti = 1) at helicity bit h
   auto spinor = [&](int anti, int h, W<R>& w) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int o = S::FB + 16 * anti + 8 * h + 2 * q;
+      const int o = S::FB + 8 * (S::NH * anti + (S::NH > 1 ? h : 0)) + 2 * q;
       w[q + 2] = cx<R>(lds[o * BLOCK + t], lds[(o + 1) * BLOCK + t]);
     }
   };
