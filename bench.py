@@ -50,7 +50,7 @@ HBM_BYTES_PER_ME = {("gg_ttxgg_fused", 32): 28180.3, ("gg_ttxgg", 32): 27656.8}
 # of a SIMD a cycle (157.3 TFLOP/s = 256 CUs x 4 SIMDs x 32 lanes x 2 x 2.4 GHz), so a wave64
 # FP32 instruction holds its SIMD for 2 cycles at that peak.  One wave issues at most one
 # instruction in 4 cycles; with two on a SIMD the kernels were measured at 1.35 in 4 cycles.
-VALU_WAVE_INSTS_PER_ME = {("gg_ttxgg", 32): 18997.4}
+VALU_WAVE_INSTS_PER_ME = {("gg_ttxgg", 32): 19049.0}
 VALU_CYCLES_PER_INST = 2
 ENGINE_HZ = 2.4e9
 METRIC = "unweighted events/sec at sigma/sigma=1e-3 and ME evals/sec, gg->ttgg on 1 MI355X"

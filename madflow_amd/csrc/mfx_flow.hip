@@ -544,12 +544,14 @@ k_flow(FlowArgs A, const float* __restrict__ P,
 // 16-column tile at a time, the widths, the heights, then the derivatives, each read into
 // registers before the next is staged.  Each output element sums the same products in the same
 // order as in k_flow: the results are equal to the last bit.  What bounds it is latency: a
-// wave's layer is a chain of products, LDS and special functions between four barriers, and
+// wave's layer is a chain of products, LDS and special functions between five barriers, and
 // neither the VALU nor the matrix cores are busy half of the time.  So it takes as many waves
 // as fit: 51 KB of LDS and 168 registers, three blocks on a CU (two with all 49 parameters
 // of a sample staged at once, 79 KB; the products of W3 are unrolled twice only, as more spills).
 // 1e6 samples of an 8-layer flow, inverse: 8 dimensions 7.14 ms in k_flow, 2.52 with two blocks on a CU,
-// 1.97 now; 11 dimensions 14.6, 3.43, 2.68 ms; 4 dimensions (6 layers) 4.45, 1.63, 1.29 ms.
+// 1.97 now; 11 dimensions 14.6, 3.43, 2.68 ms; 4 dimensions (6 layers) 4.45, 1.63, 1.29 ms.  Waves
+// idle through layer 3 and the spline unless the transformed dimensions are a multiple of
+// four: with two (4 dimensions) a layer takes 0.215 ms, with four (8) 0.246.
 constexpr int WT = 64;          // samples per block
 constexpr int WV = 4;           // waves per block
 constexpr int XP = DMAX + 1;    // row pitch of the coordinates in LDS (a sample per lane)

@@ -22,7 +22,10 @@ namespace mfx {
 
 constexpr int GEN_BLOCK = 256;
 constexpr int ACC_BLOCK = 256;
-constexpr int ACC_GRID = 1024;      // fixed: the reduction order must not depend on nev
+// The most blocks of the accumulation kernels.  Fewer events launch fewer (acc_blocks), to the same
+// sums: an event's block and the tree that merges the partials stay, and those left out would
+// have held exact zeros.
+constexpr int ACC_GRID = 1024;
 constexpr int MAXDIM = 32;
 constexpr int MAXBINS = 64;
 constexpr int ACC_PARTS = 2;      // copies of the histogram a wave, at most
@@ -627,7 +630,7 @@ __global__ void __launch_bounds__(ACC_BLOCK) k_mc_moments(int64_t nev, int nch, 
   }
 }
 
-// Sum of up to RED_T x 16 compensated partials (s, c) at q, q + stride, ..., by one block:
+// Sum of nparts compensated partials (s, c) at q, q + stride, ..., by one block:
 // thread t adds t, t + RED_T, ... in order, then the threads merge in a fixed tree, so the
 // result does not depend on scheduling.  Thread 0 returns the sum.
 constexpr int RED_T = 256;

@@ -913,6 +913,10 @@ int64_t ordered_ws_per_row(int precision) {
 // second wave of a SIMD out (t t~ g g g FP32, 1,000 events: 1,056 us against 610 us with two); four
 // and eight are within the scatter of the rounds they end in (1,000 events: 652 and 638 us; 2,500
 // events: 1,437 and 1,493 us against 1,711 us; 257 events: 296 and 273 us against 267 us).
+// FP64 holds one wave a SIMD, but two ranges for each are as often the better split as one: with
+// one, two and four, t t~ g g 500 events 30, 35 and 35 us, 1,000 47, 57 and 54, 2,500 125, 109 and 104, 4,000
+// 163, 137 and 143, 8,000 254, 282 and 260; t t~ g g g 500 events 720, 876 and 756, 2,500 4,770, 3,830 and
+// 3,390, from 4,000 on the same.
 constexpr int ORDERED_WAVES = 2;
 
 // (tile, rows) items per wave slot of k_colour_mfma: t t~ g g g FP32, 50,000 events, 27.2 ms a call
