@@ -426,14 +426,12 @@ __global__ void __launch_bounds__(256) k_matrix_hel(SmatrixArgs a) {
 }
 
 // Whether k_smatrix is built: for the processes that k_smatrix_rows does not take, and for FP32 with
-// few pairs of rows or one wave a SIMD, where its full rounds of 256 events a CU are the faster form:
-// from `fewest` of them on, if the last leaves less than 1 / slack of the others empty.
+// few pairs of rows, where its full rounds of 256 events a CU are the faster form: from `fewest` of
+// them on, if the last leaves less than 1 / slack of the events' number empty.
 template <class T, class R> struct KeepsEvents {
   static constexpr int pairs = T::NCOMB / (T::FILTERED ? 4 : 2);
-  static constexpr bool value =
-      !SideBySide<T, R>::value || (StableForms<R>::value && (pairs < 16 || RowsWaves<T, R>::value == 1));
-  static constexpr int fewest = pairs >= 16 ? 1 : (T::NCOLOR > 2 ? 2 : 3);
-  static constexpr int slack = pairs >= 16 ? 40 : (T::NCOLOR > 2 ? 10 : 20);
+  static constexpr bool value = !SideBySide<T, R>::value || (StableForms<R>::value && pairs < 16);
+  static constexpr int fewest = T::NCOLOR > 2 ? 2 : 3, slack = T::NCOLOR > 2 ? 10 : 20;
 };
 
 struct ProcessEntry {
@@ -463,9 +461,10 @@ struct ProcessEntry {
 // 72.2 and 69.5, 1e6 262 and 252; u u~ > t t~ 131,072 14.5 and 14.7, 262,144 25.1 and 24.2, 1e6 85 and 79;
 // u u~ > t t~ g 100,000 56 and 61, 120,000 63.7 and 60.9, 196,608 94.5 and 84.6, 225,000 109.7 and 110.6, 262,144
 // 125 and 111, 1e6 473 and 398; u g > t t~ u 100,000 57 and 63, 120,000 64.7 and 62.6, 262,144 127 and 117.
-// With 16 pairs at one wave a SIMD (u u~ > t t~ g g) k_smatrix takes 2% less for an event: 65,536 events 316
-// and 311, 400,000 1,970 and 2,170, 983,040 4,720 and 4,630, 1e6 4,880 and 4,940, 3e6 14,500 and 14,200.
-// At two waves (t t~ g) it takes longer (1e6 events 1,840 and 2,340).
+// With 16 pairs it is not built: it takes longer at two waves a SIMD (t t~ g, 1e6 events 1,840 and 2,340),
+// and at one (u u~ > t t~ g g) 400,000 events 1,970 and 2,170, 1e6 4,880 and 4,940, against 2% less where its rounds
+// are full (983,040 events 4,720 and 4,630, 3e6 14,500 and 14,200).  Built beside them, it cost the FP64 rows
+// of that process 1.5%, which then lie elsewhere in memory (87 KB of instructions).
 template <class T, class R>
 int events_per_block(int64_t nev) {
   constexpr int pairs = KeepsEvents<T, R>::pairs;
@@ -476,8 +475,7 @@ int events_per_block(int64_t nev) {
   if constexpr (KeepsEvents<T, R>::value) {
     constexpr int fewest = KeepsEvents<T, R>::fewest, slack = KeepsEvents<T, R>::slack;
     const int64_t round = 256ll * cus, rounds = (nev + round - 1) / round;
-    if (pairs < 16 && rounds > 4) return 0;
-    if (rounds >= fewest && slack * (rounds * round - nev) <= nev) return 0;
+    if (rounds > 4 || (rounds >= fewest && slack * (rounds * round - nev) <= nev)) return 0;
   }
   int best = 64;
   int64_t least = INT64_MAX;

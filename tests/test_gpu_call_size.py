@@ -54,8 +54,7 @@ def test_matrix_elements_of_split_rows(dev, name, large, precision):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name,sizes", [("uux_ttxgg", (63000, 65000, 65536, 65537, 131072)),
-                                        ("uux_ttxg", (110000, 120000, 131073, 240000, 262145)),
+@pytest.mark.parametrize("name,sizes", [("uux_ttxg", (110000, 120000, 131073, 240000, 262145)),
                                         ("ug_ttxu", (119000, 119200, 131073)),
                                         ("gg_ttx", (131072, 187000, 188000, 196609))])
 def test_rows_side_by_side_or_in_turn(dev, name, sizes):
